@@ -4,13 +4,15 @@
 // contiguous, 4 KiB at 16 keys of 128 dims), token j in physical page
 // page_table[j / page_size] at slot j % page_size.
 //
-//  * Block (b, g) takes keys [1024 b, 1024 b + 1024) of KV head g; each of its 4 waves 256
-//    keys, as pairs of 16-key tiles (a tile is one MFMA tile, inside one page: one
+//  * Block (b, g) takes keys [128 NP b, 128 NP (b + 1)) of KV head g; each of its 4 waves
+//    32 NP keys, as NP pairs of 16-key tiles (a tile is one MFMA tile, inside one page: one
 //    contiguous 4 KiB run of K and one of V). K and V of a tile stream once for all G
 //    query heads; the next pair's loads are in flight while the current one is reduced.
-//    At 32 Ki keys and 8 KV heads that is 256 blocks, one a CU, and 32 partials a KV head
-//    for the merge (measured against 64 keys a wave: 29.4 against 31.8 us a step; 128:
-//    30.5; 512 keys a wave, or 8-wave blocks, or two and three pairs in flight: slower).
+//    attn_pairs picks NP so that the grid fills the chip once: at 32 Ki keys and 8 KV heads
+//    NP = 8, 256 blocks, one a CU, and 32 partials a KV head for the merge (512 keys a wave,
+//    8-wave blocks, or two and three pairs in flight: slower); a short sequence takes NP = 1,
+//    its waves one round of loads each (700 keys over 8 KV heads: 8.0 us a step, 15.3 at
+//    NP = 8, whose 8 blocks left 248 CUs idle).
 //  * Scores S^T = K . Q^T on bf16 MFMA (v_mfma_f32_16x16x32_bf16; products exact, fp32
 //    accumulate): keys are the M side, so K loads need head_dim contiguous per lane
 //    (the layout in memory) and each lane ends with 4 keys of one head, which keeps the
@@ -34,15 +36,16 @@
 namespace oom {
 
 constexpr int AW = 4;           // waves per block
-constexpr int AKW = 256;        // keys per wave
-constexpr int AKB = AW * AKW;   // keys per block
+constexpr int AKB = AW * 256;   // keys per block of the coarsest split
 constexpr int AG = 8;           // query heads per KV head (at most)
 constexpr int A_MAXB = 8192;    // blocks a KV head (8 Mi keys): the merge's weights sit in LDS
 constexpr int A_BUF_FLAGS = 0x00020000;
 constexpr int A_OOB = 0x7ffffff0;
 constexpr int A_BUF_SC1 = 16;
 
+typedef __bf16 abf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 abf16x8 __attribute__((ext_vector_type(8)));
+typedef float af32x2 __attribute__((ext_vector_type(2)));
 typedef float af32x4 __attribute__((ext_vector_type(4)));
 
 struct AttnArgs {
@@ -161,9 +164,9 @@ __device__ __forceinline__ float group_sum(float v) {
     return __uint_as_float(r2[0]) + __uint_as_float(r2[1]);
 }
 
-template <int D, int QDT, int ODT>
+template <int D, int QDT, int ODT, int NP>
 __global__ void __launch_bounds__(AW * 64) attn_decode_kernel(AttnArgs a) {
-    constexpr int NS = D / 32, NP = AKW / 32, NB = D / 16;
+    constexpr int NS = D / 32, NB = D / 16;
     static_assert(D == 128 && AW * VT_WORDS >= AW * AG * D, "the V areas hold the block merge afterwards");
     // the waves' transposed V areas; after the key loop, the block merge's accumulators
     __shared__ __align__(16) uint32_t vts[AW * VT_WORDS];
@@ -172,7 +175,7 @@ __global__ void __launch_bounds__(AW * 64) attn_decode_kernel(AttnArgs a) {
     const int lane = threadIdx.x & 63, tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = blockIdx.y, b = blockIdx.x, G = a.G;
-    const int kbase = b * AKB + wave * AKW;
+    const int kbase = (b * AW + wave) * 32 * NP;
     uint32_t* const vt = vts + wave * VT_WORDS;
     // Q^T as the MFMA B operand: column = head l % 16 (zero past G), head_dim 32 s + 8 (l / 16) .. + 8
     constexpr int NQ = QDT == OOM_F32 ? 3 : 1;
@@ -189,22 +192,25 @@ __global__ void __launch_bounds__(AW * 64) attn_decode_kernel(AttnArgs a) {
                                     : make_uint4(0, 0, 0, 0);
                 qb[0][s] = __builtin_bit_cast(abf16x8, v);
             } else {
-                float f[8];
+                // two 16-byte loads whatever the head (head 0's for a head past G), then the
+                // select: with each load under the test, the compiler moved it into a branch
+                // behind the wait of the one before (32 round trips, 4 us a call)
+                const float4* qp = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(a.q) + qi);
+                const float4 v0 = qp[0], v1 = qp[1];
+                float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
 #pragma unroll
-                for (int e = 0; e < 8; e++) f[e] = hok ? reinterpret_cast<const float*>(a.q)[qi + e] : 0.0f;
+                for (int e = 0; e < 8; e++) f[e] = hok ? f[e] : 0.0f;
 #pragma unroll
                 for (int term = 0; term < 3; term++) {
-                    uint16_t hb[8];
+                    uint32_t wv[4];
 #pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        hb[e] = f32_to_bf16(f[e]);
-                        f[e] -= bf16_to_f32(hb[e]);  // exact: the remainder of a round to nearest
+                    for (int e = 0; e < 4; e++) {
+                        const af32x2 pf = {f[2 * e], f[2 * e + 1]};
+                        wv[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pf, abf16x2));  // RNE
+                        f[2 * e] -= __uint_as_float(wv[e] << 16);  // exact: the remainder of a round to nearest
+                        f[2 * e + 1] -= __uint_as_float(wv[e] & 0xffff0000u);
                     }
-                    uint4 v;
-                    v.x = hb[0] | (uint32_t(hb[1]) << 16);
-                    v.y = hb[2] | (uint32_t(hb[3]) << 16);
-                    v.z = hb[4] | (uint32_t(hb[5]) << 16);
-                    v.w = hb[6] | (uint32_t(hb[7]) << 16);
+                    const uint4 v = make_uint4(wv[0], wv[1], wv[2], wv[3]);
                     qb[term][s] = __builtin_bit_cast(abf16x8, v);
                 }
             }
@@ -272,8 +278,6 @@ __global__ void __launch_bounds__(AW * 64) attn_decode_kernel(AttnArgs a) {
         abf16x8 pa[3];
 #pragma unroll
         for (int term = 0; term < 3; term++) {
-            typedef __bf16 abf16x2 __attribute__((ext_vector_type(2)));
-            typedef float af32x2 __attribute__((ext_vector_type(2)));
             uint32_t wv[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
@@ -439,24 +443,65 @@ __global__ void __launch_bounds__(128) attn_merge_kernel(AttnArgs a) {
 
 static size_t a_al256(size_t v) { return (v + 255) & ~size_t(255); }
 
+// Splits of a KV head's keys: blocks of 4 waves with 32 NP keys a wave, NP = 1, 2, 4 or 8
+// pairs of tiles. One wave's pairs follow each other (about 1.4 us each: one pair is in
+// flight), so the finest split that still fits the chip is the fastest: at 64 / 8 heads, us a
+// step, NP = 1, 2, 4, 8 by keys
+//     1000:  8.0,  9.1, 12.1, 15.3      4096:  9.7, 10.0, 12.5, 18.7
+//     8192: 13.3, 12.1, 13.2, 18.7     16384: 17.9, 17.4, 16.6, 19.4
+//    32768: 49.1, 31.9, 30.5, 29.5     65536: 90.9, 70.9, 54.5, 54.2
+// so NP is the smallest whose blocks number at most A_FILL over all KV heads (one a CU; the
+// rows' best ends there: 4096 keys are 256 blocks at NP = 1, 8192 at NP = 2, 16384 at NP = 4)
+// and whose partials a KV head the merge takes in one round (at 1 KV head and 32768 keys, 256
+// partials: 25.3 us against 10.8 for 128 at NP = 2). Up to 256 keys one block holds the KV
+// head and no merge is launched (200 keys: 5.9 us at NP = 2 against 7.9 at NP = 1 and 13.7 at
+// NP = 8).
+constexpr int A_FILL = 256;  // blocks over all KV heads
+constexpr int A_ROUND = 128; // partials a KV head the merge loads at once
+
 struct AttnWs {
-    size_t part, total;
+    size_t least, total;  // what the coarsest split needs, and what every split at up to kv_len keys fits in
 };
 
+static size_t attn_part_bytes(int blocks, int kv_heads, int d) {
+    return a_al256((size_t)kv_heads * blocks * (2 * AG + AG * (size_t)d) * sizeof(float));
+}
+
+// A sequence that grows within one workspace: the finer splits of shorter sequences take at
+// most min(A_ROUND, A_FILL / kv_heads) blocks a KV head, so `total` never falls with kv_len.
 static AttnWs attn_ws(int kv_len, int kv_heads, int d) {
     AttnWs w;
-    const int bph = (int)cdiv(kv_len, AKB);
-    w.part = 0;
-    w.total = a_al256((size_t)kv_heads * (bph > 1 ? bph : 1) * (2 * AG + AG * (size_t)d) * sizeof(float));
+    const int coarse = (int)cdiv(kv_len, AKB);
+    const int fine = std::min((int)cdiv(kv_len, 128), std::min(A_ROUND, A_FILL / kv_heads));
+    w.least = attn_part_bytes(coarse, kv_heads, d);
+    w.total = attn_part_bytes(std::max(coarse, fine), kv_heads, d);
     return w;
 }
 
+// Pairs of tiles a wave (NP): the rule above, within the workspace at hand (one sized for the
+// coarsest split alone still serves).
+static int attn_pairs(int kv_len, int kv_heads, int d, size_t ws_bytes) {
+    for (int np = kv_len <= 128 ? 1 : kv_len <= 256 ? 2 : 1; np < 8; np *= 2) {
+        const int64_t blocks = cdiv(kv_len, 128 * np);
+        if (blocks == 1 || (blocks <= A_ROUND && blocks * kv_heads <= A_FILL &&
+                            attn_part_bytes((int)blocks, kv_heads, d) <= ws_bytes))
+            return np;
+    }
+    return 8;
+}
+
 template <int D, int QDT, int ODT>
-static int launch_attn_t(const AttnArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL((attn_decode_kernel<D, QDT, ODT>), dim3(a.bph, a.Hkv), dim3(AW * 64), 0, st, a);
+static int launch_attn_t(const AttnArgs& a, int np, hipStream_t st) {
+    const dim3 grid(a.bph, a.Hkv), block(AW * 64);
+    switch (np) {
+        case 1: hipLaunchKernelGGL((attn_decode_kernel<D, QDT, ODT, 1>), grid, block, 0, st, a); break;
+        case 2: hipLaunchKernelGGL((attn_decode_kernel<D, QDT, ODT, 2>), grid, block, 0, st, a); break;
+        case 4: hipLaunchKernelGGL((attn_decode_kernel<D, QDT, ODT, 4>), grid, block, 0, st, a); break;
+        default: hipLaunchKernelGGL((attn_decode_kernel<D, QDT, ODT, 8>), grid, block, 0, st, a); break;
+    }
     if (a.bph > 1) {
         if (int rc = launched("oom_attn_decode_paged")) return rc;
-        hipLaunchKernelGGL((attn_merge_kernel<D, ODT>), dim3(a.Hkv, a.G, a.bph <= 128 ? 4 : 1), dim3(128), 0, st, a);
+        hipLaunchKernelGGL((attn_merge_kernel<D, ODT>), dim3(a.Hkv, a.G, a.bph <= A_ROUND ? 4 : 1), dim3(128), 0, st, a);
     }
     return launched("oom_attn_decode_paged");
 }
@@ -486,7 +531,7 @@ extern "C" int oom_attn_decode_paged(const void* q, int q_dtype, const uint16_t*
     OOM_REQUIRE(aligned(q, 16) && aligned(k_pages, 16) && aligned(v_pages, 16),
                 "oom_attn_decode_paged: q, k_pages and v_pages must be 16-byte aligned");
     const AttnWs w = attn_ws(kv_len, kv_heads, d);
-    if (!ws || ws_bytes < w.total)
+    if (!ws || ws_bytes < w.least)
         return fail(OOM_ERR_WORKSPACE, "oom_attn_decode_paged: workspace smaller than oom_attn_decode_workspace_size()");
     OOM_REQUIRE(aligned(ws, 256), "oom_attn_decode_paged: workspace must be 256-byte aligned");
     uint8_t* base = reinterpret_cast<uint8_t*>(ws);
@@ -500,14 +545,15 @@ extern "C" int oom_attn_decode_paged(const void* q, int q_dtype, const uint16_t*
     a.kv_len = kv_len;
     a.Hkv = kv_heads;
     a.G = heads / kv_heads;
-    a.bph = (int)cdiv(kv_len, AKB);
+    const int np = attn_pairs(kv_len, kv_heads, d, ws_bytes);
+    a.bph = (int)cdiv(kv_len, 128 * np);
     a.scale = scale;
     a.out = out;
-    a.part = reinterpret_cast<float*>(base + w.part);
+    a.part = reinterpret_cast<float*>(base);
     hipStream_t st = as_stream(stream);
     if (q_dtype == OOM_BF16)
-        return out_dtype == OOM_BF16 ? launch_attn_t<128, OOM_BF16, OOM_BF16>(a, st)
-                                     : launch_attn_t<128, OOM_BF16, OOM_F32>(a, st);
-    return out_dtype == OOM_BF16 ? launch_attn_t<128, OOM_F32, OOM_BF16>(a, st)
-                                 : launch_attn_t<128, OOM_F32, OOM_F32>(a, st);
+        return out_dtype == OOM_BF16 ? launch_attn_t<128, OOM_BF16, OOM_BF16>(a, np, st)
+                                     : launch_attn_t<128, OOM_BF16, OOM_F32>(a, np, st);
+    return out_dtype == OOM_BF16 ? launch_attn_t<128, OOM_F32, OOM_BF16>(a, np, st)
+                                 : launch_attn_t<128, OOM_F32, OOM_F32>(a, np, st);
 }

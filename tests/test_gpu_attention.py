@@ -107,3 +107,49 @@ def test_attention_convex_and_page_order(hip):
     got2 = run(hip, q, k2, v2, perm[table].astype(np.int32), kv_len, 0.2, torch.float32)
     np.testing.assert_array_equal(got, got2)
 
+
+
+@pytest.mark.parametrize("H,Hkv,kv_len,page,qdt", [
+    (8, 1, 128, 16, "bf16"), (16, 2, 129, 32, "f32"), (6, 1, 256, 16, "f32"),  # one block: NP 1, then 2
+    (8, 1, 257, 64, "bf16"), (32, 8, 700, 16, "bf16"),                         # three and six blocks of 128 keys
+    (64, 8, 4096, 16, "f32"), (64, 8, 4097, 16, "bf16"),                       # 256 blocks at NP 1; past it NP 2
+    (32, 8, 8193, 32, "bf16"), (16, 8, 16385, 16, "f32"),                      # NP 4, NP 8
+    (4, 1, 16385, 16, "bf16"), (4, 1, 32769, 16, "f32"),                       # past 128 partials at NP 1, at NP 2
+])
+def test_attention_split_sizes(hip, H, Hkv, kv_len, page, qdt):
+    """Every split a KV head's keys can take, at the sizes where the rule changes, against f64
+    (the file's 1e-4 bar) and against the coarsest split, which a workspace of its size gets
+    (the two differ in summation order alone: 2e-6 of the largest output, 16 times the 2^-23
+    of one rounding)."""
+    import torch
+
+    print(f"attention split H={H} Hkv={Hkv} kv_len={kv_len} page={page} q={qdt}", flush=True)
+    D = 128
+    q, k, v, table = synth.paged_attention_case(23 + kv_len, H, Hkv, D, kv_len, page)
+    qf = oracle.bf16_to_f32(q)
+    qd = torch.from_numpy(qf).cuda()
+    if qdt == "bf16":
+        qd = qd.to(torch.bfloat16)
+    kd, vd = (torch.from_numpy(t.view(np.int16)).view(torch.bfloat16).cuda() for t in (k, v))
+    td = torch.from_numpy(table).cuda()
+    least = (Hkv * -(-kv_len // 1024) * (16 + 8 * D) * 4 + 255) // 256 * 256
+    full = hip.attn_decode_workspace_size(kv_len, H, Hkv, D)
+    assert full >= least
+    outs = []
+    for size in (full, least):
+        ws = torch.zeros(size, dtype=torch.uint8, device="cuda")
+        out = torch.empty((H, D), dtype=torch.float32, device="cuda")
+        hip.attn_decode_paged(qd, kd, vd, td, kv_len, 0.09, out, ws)
+        outs.append(out.cpu().numpy())
+    with pytest.raises(hip.OomError, match="workspace"):
+        hip.attn_decode_paged(qd, kd, vd, td, kv_len, 0.09, out, ws[:least - 256])
+    want = synth.f64_attention(qf, k, v, table, page, kv_len, H, Hkv, D, 0.09)
+    assert np.abs(outs[0] - want).max() < 1e-4
+    assert np.abs(outs[0] - outs[1]).max() < 2e-6 * np.abs(want).max()
+
+
+def test_attention_workspace_grows_with_the_sequence(hip):
+    """A workspace made for a length serves every shorter one."""
+    for Hkv in (1, 3, 8, 64, 300):
+        sizes = [hip.attn_decode_workspace_size(n, Hkv, Hkv, 128) for n in range(1, 70000, 61)]
+        assert sizes == sorted(sizes)
