@@ -57,6 +57,7 @@ __device__ __forceinline__ float kv_sign(int i) { return (((unsigned)i * 2654435
 // and add fuse here (fp contract off): the format's arithmetic rounds each product (a
 // decoded level times its scale, a square) before it enters a butterfly or a sum.
 constexpr int TR_WAVES = 4;  // waves a block of the row kernels
+constexpr int TQ_OOB = 0x70000000;  // an offset past every buffer here: loads read 0
 
 // Walsh-Hadamard butterflies over the row in the format's stage order h = 1, 2, ..., D / 2,
 // each pair (i, i + h) becoming (s_i + s_{i+h}, s_i - s_{i+h}): stages 1 and 2 inside the
@@ -151,15 +152,23 @@ __global__ void __launch_bounds__(64 * TR_WAVES) kv_append_kernel(const float* _
                                                                  int64_t rows, int bits,
                                                                  const float* __restrict__ lv_all) {
 #pragma clang fp contract(off)
-    __shared__ float lv[256];
+    __shared__ float lv[64 * TR_WAVES];
+    static_assert(64 * TR_WAVES >= 256, "one level a thread");
     const int lane = threadIdx.x & 63, n = 1 << bits;
-    for (int t = threadIdx.x; t < n; t += blockDim.x) lv[t] = lv_all[codebook_offset(bits) + t];
     int l;
-    const int64_t r = row_of<D>(lane, l);
+    const int64_t r = row_of<D>(lane, l), r0 = (int64_t)blockIdx.x * TR_WAVES * (256 / D);
     const bool ok = r < rows;
+    // the row and the levels in one round of loads (buffer loads, a row or level past the end
+    // reading zeros; dwords: the ABI asks 4-byte alignment only): one token's append is the
+    // latency of its loads, and the levels' loop had waited before the row's loads went out
+    const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(src + r0 * D), (short)0, TR_WAVES * 256 * 4, BUF_FLAGS);
+    const __amdgpu_buffer_rsrc_t lr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(lv_all), (short)0, TQ_LEVELS * 4, BUF_FLAGS);
     float y[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) y[i] = ok ? src[r * D + 4 * l + i] : 0.0f;
+    for (int i = 0; i < 4; i++) y[i] = ldf(sr, ok ? ((int)(r - r0) * D + 4 * l + i) * 4 : TQ_OOB);
+    lv[threadIdx.x] = ldf(lr, (int)threadIdx.x < n ? (codebook_offset(bits) + (int)threadIdx.x) * 4 : TQ_OOB);
 #pragma unroll
     for (int i = 0; i < 4; i++) y[i] *= kv_sign(4 * l + i);
     row_wht<D>(y, lane);
@@ -173,23 +182,33 @@ __global__ void __launch_bounds__(64 * TR_WAVES) kv_append_kernel(const float* _
     const __half hs = __float2half(sqrtf(ss / 32.0f));  // round to nearest even
     const float sc = __half2float(hs);
     __syncthreads();  // the levels are in LDS
+    // idx: the last level at or below u among the first n - 1 (0 if none), or its upper
+    // neighbour if that one is nearer. The bisection's steps take the four coordinates
+    // together (their LDS reads in flight at once), largest power of two first: one token's
+    // append is these dependent reads (4 x 7 of them one after the other before)
     int idx[4];
+    float u[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const float u = sc > 0.0f ? y[i] / sc : 0.0f;
-        int lo = 0, hi = n - 1;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (lv[mid] <= u) lo = mid;
-            else hi = mid;
-        }
-        idx[i] = fabsf(u - lv[lo]) <= fabsf(u - lv[hi]) ? lo : hi;
+        u[i] = sc > 0.0f ? y[i] / sc : 0.0f;
+        idx[i] = 0;
     }
+    for (int s = n >> 1; s > 0; s >>= 1) {
+        float at[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) at[i] = lv[min(idx[i] + s, n - 1)];
+#pragma unroll
+        for (int i = 0; i < 4; i++) idx[i] = idx[i] + s <= n - 2 && at[i] <= u[i] ? idx[i] + s : idx[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) idx[i] = fabsf(u[i] - lv[idx[i]]) <= fabsf(u[i] - lv[idx[i] + 1]) ? idx[i] : idx[i] + 1;
     // word j of the block: bit t = 4 (l % 8) + i is bit j of coordinate t's code; the 8
-    // lanes OR their nibbles together and lane l % 8 == j keeps word j
+    // lanes OR their nibbles together and lane l % 8 == j keeps word j (unrolled, so the words'
+    // exchanges overlap)
     const int lb = l & 7, b = l >> 3;
     uint32_t mine = 0;
-    for (int j = 0; j < bits; j++) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
         uint32_t nib = 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) nib |= (uint32_t)((idx[i] >> j) & 1) << i;
@@ -328,10 +347,7 @@ __global__ void __launch_bounds__(TQ_MASK_THREADS) mask_compact_kernel(const uin
 // 1.5 VALU operations a coordinate), then looks the level up in an LDS copy of the
 // codebook and multiplies by the block's scale -- the same f32 product as the reference's
 // per-coordinate decode.
-constexpr int TT_WAVES = 8;  // waves a block: two a SIMD, so one wave's MFMAs overlap the other's decoding
-constexpr int TT_GPW = 2;    // groups of 16 keys a wave is sized for (one a round)
 constexpr int TT_QS = 260;   // LDS row stride (floats) of a query head
-constexpr int TQ_OOB = 0x70000000;  // an offset past every buffer here: loads read 0
 constexpr int TC_THREADS = 1024;    // combine block: 4 slices of the partials x 256 coordinates
 constexpr int TC_BATCH = 32;        // partials a combine thread loads at once
 
@@ -596,11 +612,12 @@ __device__ __forceinline__ uint32_t tq_mask_byte(__amdgpu_buffer_rsrc_t mr, int 
 }
 __device__ __forceinline__ uint32_t tq_ballot(uint32_t b) { return (uint32_t)__ballot(b != 0); }
 
+template <int TW>
 struct TqLds {
     float lvk[256], lvv[256];                                  // codebooks of the K and V rows
     __attribute__((aligned(16))) float qsp[16][TT_QS];          // queries in score-step order
-    float red[TT_WAVES][TQ_G][2];                               // each wave's max and sum a head
-    __attribute__((aligned(16))) float osum[TT_WAVES][TQ_G][TQ_D];  // each wave's rescaled output
+    float red[TW][TQ_G][2];                                     // each wave's max and sum a head
+    __attribute__((aligned(16))) float osum[TW][TQ_G][TQ_D];  // each wave's rescaled output
 };
 
 // The online softmax keeps a reference maximum per head and moves it only when a score
@@ -608,13 +625,13 @@ struct TqLds {
 // the accumulated output is rescaled rarely instead of every round.
 constexpr float TQ_TAU = 8.0f;
 
-template <int KB, int VB>
-__global__ void __launch_bounds__(TT_WAVES * 64) attn_turbo_kernel(TurboArgs a) {
+template <int KB, int VB, int TW>
+__global__ void __launch_bounds__(TW * 64) attn_turbo_kernel(TurboArgs a) {
     constexpr bool ROT = KB != 0;
     constexpr int D = TQ_D, G = TQ_G;
     // one LDS object with the codebooks first: their addresses are constants that fold
     // into the lookups' offset field
-    __shared__ TqLds sm;
+    __shared__ TqLds<TW> sm;
     float* lvk = sm.lvk;
     float* lvv = sm.lvv;
     float(*qsp)[TT_QS] = sm.qsp;
@@ -624,7 +641,7 @@ __global__ void __launch_bounds__(TT_WAVES * 64) attn_turbo_kernel(TurboArgs a) 
     const int kvh = blockIdx.y;
     const int kb = KB >= 0 ? KB : a.kb, vb = VB >= 0 ? VB : a.vb;
     const int krb = kv_row_bytes(D, kb), vrb = kv_row_bytes(D, vb);
-    const int W = a.nblk * TT_WAVES, wv = blockIdx.x * TT_WAVES + wave;
+    const int W = a.nblk * TW, wv = blockIdx.x * TW + wave;
     const int ngroups = (a.kv_len + 15) >> 4;
     const __amdgpu_buffer_rsrc_t mr = tq_rsrc(a.mask, a.kv_len);
     const __amdgpu_buffer_rsrc_t kr = tq_rsrc(a.k, a.kv_len * a.Hkv * krb);
@@ -638,10 +655,11 @@ __global__ void __launch_bounds__(TT_WAVES * 64) attn_turbo_kernel(TurboArgs a) 
     const uint32_t b1 = tq_mask_byte(mr, a.kv_len, ngroups, wv, W, 1, lane);
     // wave w rotates heads w and w + 8 (rows 12 .. 15 are zero); lane l holds coordinates
     // 4 l .. 4 l + 3
-    uint4 qh[2];
+    constexpr int NJ = 16 / TW;
+    uint4 qh[NJ];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int h = wave + TT_WAVES * j;
+    for (int j = 0; j < NJ; j++) {
+        const int h = wave + TW * j;
         qh[j] = ld16(qr, h < G ? (h * D + 4 * lane) * 4 : TQ_OOB);
     }
     float lk = 0.0f, lv = 0.0f;
@@ -668,7 +686,7 @@ __global__ void __launch_bounds__(TT_WAVES * 64) attn_turbo_kernel(TurboArgs a) 
     // l ^ 32); the 1/16 normalisation is folded into the score scale (a power of two:
     // exact). The result goes to LDS in the order the score steps read it.
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
+    for (int j = 0; j < NJ; j++) {
         float x[4] = {__uint_as_float(qh[j].x), __uint_as_float(qh[j].y), __uint_as_float(qh[j].z),
                       __uint_as_float(qh[j].w)};
         if constexpr (ROT) {
@@ -684,12 +702,12 @@ __global__ void __launch_bounds__(TT_WAVES * 64) attn_turbo_kernel(TurboArgs a) 
                 const bool upper = lane & o;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float y = __shfl_xor(x[i], o);
+                    const float y = lane_xor_n(x[i], o, lane);
                     x[i] = upper ? y - x[i] : x[i] + y;
                 }
             }
         }
-        const int h = wave + TT_WAVES * j;
+        const int h = wave + TW * j;
 #pragma unroll
         for (int i = 0; i < 4; i++) qsp[h][tq_qperm(4 * lane + i)] = x[i];
     }
@@ -769,7 +787,7 @@ __global__ void __launch_bounds__(TT_WAVES * 64) attn_turbo_kernel(TurboArgs a) 
         if (h < G) {
             float M = -INFINITY;
 #pragma unroll
-            for (int w = 0; w < TT_WAVES; w++) M = fmaxf(M, red[w][h][0]);
+            for (int w = 0; w < TW; w++) M = fmaxf(M, red[w][h][0]);
             const float mw = red[wave][h][0];
             const float f = mw == -INFINITY ? 0.0f : __expf(mw - M);
 #pragma unroll
@@ -785,15 +803,15 @@ __global__ void __launch_bounds__(TT_WAVES * 64) attn_turbo_kernel(TurboArgs a) 
         const int h = u / D, c = u % D;
         float s = 0.0f;
 #pragma unroll
-        for (int w = 0; w < TT_WAVES; w++) s += osum[w][h][c];
+        for (int w = 0; w < TW; w++) s += osum[w][h][c];
         part[u] = s;
     }
     if (tid < G) {
         float M = -INFINITY, L = 0.0f;
 #pragma unroll
-        for (int w = 0; w < TT_WAVES; w++) M = fmaxf(M, red[w][tid][0]);
+        for (int w = 0; w < TW; w++) M = fmaxf(M, red[w][tid][0]);
 #pragma unroll
-        for (int w = 0; w < TT_WAVES; w++) {
+        for (int w = 0; w < TW; w++) {
             const float mw = red[w][tid][0];
             if (mw != -INFINITY) L += __expf(mw - M) * red[w][tid][1];
         }
@@ -952,28 +970,44 @@ static bool kv_row_shape(int d, int bits) {
     return d >= 32 && d % 32 == 0 && d <= TQ_MAXD && (bits == 0 || ((d & (d - 1)) == 0 && bits >= 2 && bits <= 8));
 }
 
-// Blocks a KV head of the decode attention: enough that every wave has TT_GPW groups of
-// 16 keys, at most 256 blocks over all KV heads (one a CU).
-static int turbo_blocks(int kv_len, int kv_heads) {
-    const int groups = (kv_len + 15) / 16;
-    const int want = (groups + TT_WAVES * TT_GPW - 1) / (TT_WAVES * TT_GPW);
-    return std::max(1, std::min(want, std::max(1, 256 / kv_heads)));
+// How a KV head's keys are dealt: blocks of `waves` waves, `blocks` of them a KV head. A wave's
+// groups follow each other (about 4 us each: 128 fp32 MFMAs and the decoding between them), so
+// every wave takes one group as long as the grid then has a block a CU or fewer:
+//   - blocks of 4 waves, one a SIMD, while ceil(groups / 4) blocks a KV head make at most
+//     TT_FILL in all; past that two of them share a CU (9001 keys, 2 KV heads, us a call with
+//     the combine: 27.7 as 282 blocks of 4 waves, 18.7 as 142 of 8);
+//   - else blocks of 8 waves, at most TT_FILL in all, their waves taking more groups from there;
+//   - fp32 rows (no decoding for a second wave's MFMAs to hide behind) keep 4 waves up to two
+//     groups a wave: 17.0 us against 19.4 at 9001 keys, 2 KV heads.
+// Before, every wave was sized for two groups on blocks of 8: us a call then and now, k8v6, all
+// keys visible, 2 KV heads: 24.4 -> 15.5 at 700 keys, 24.5 -> 16.1 at 4500, 24.7 -> 18.7 at
+// 9001, 24.8 -> 19.8 at 16384, 26.2 at 32768 (the same split).
+constexpr int TT_FILL = 256;
+
+struct TurboSplit {
+    int waves, blocks;
+};
+
+static TurboSplit turbo_split(int kv_len, int kv_heads, bool fp32) {
+    const int groups = (kv_len + 15) / 16, most = std::max(1, TT_FILL / kv_heads);
+    for (int per = 4; per <= (fp32 ? 8 : 4); per += 4)
+        if ((groups + per - 1) / per <= most) return {4, (groups + per - 1) / per};
+    return {8, std::min((groups + 7) / 8, most)};
 }
 
-struct TurboWs {
-    size_t part, ml, total;
-    int nblk;
-};
+// Two groups a wave on blocks of 8 waves: the fewest partials, for a workspace with room for
+// no more.
+static TurboSplit turbo_split_least(int kv_len, int kv_heads) {
+    const int groups = (kv_len + 15) / 16;
+    return {8, std::max(1, std::min((groups + 15) / 16, std::max(1, TT_FILL / kv_heads)))};
+}
 
 static size_t t_al256(size_t v) { return (v + 255) & ~size_t(255); }
 
-static TurboWs turbo_ws(int kv_heads, int kv_len) {
-    TurboWs w;
-    w.nblk = turbo_blocks(kv_len, kv_heads);
-    w.part = 0;
-    w.ml = t_al256((size_t)kv_heads * w.nblk * TQ_G * TQ_D * 4);
-    w.total = w.ml + t_al256((size_t)kv_heads * w.nblk * TQ_G * 2 * 4);
-    return w;
+// Offset of the maxima and sums behind the partial outputs, and the bytes of both.
+static size_t turbo_ml(int kv_heads, int blocks) { return t_al256((size_t)kv_heads * blocks * TQ_G * TQ_D * 4); }
+static size_t turbo_bytes(int kv_heads, int blocks) {
+    return turbo_ml(kv_heads, blocks) + t_al256((size_t)kv_heads * blocks * TQ_G * 2 * 4);
 }
 
 }  // namespace oom
@@ -1075,9 +1109,22 @@ extern "C" int oom_mask_compact(const uint8_t* mask, int32_t* sel, int n, void* 
     return launched("oom_mask_compact");
 }
 
+namespace oom {
+
+template <int TW>
+static void launch_turbo(const TurboArgs& a, hipStream_t st) {
+    const dim3 grid((unsigned)a.nblk, (unsigned)a.Hkv), block(TW * 64);
+    if (a.kb == 0) hipLaunchKernelGGL((attn_turbo_kernel<0, 0, TW>), grid, block, 0, st, a);
+    else if (a.kb == 8 && a.vb == 6) hipLaunchKernelGGL((attn_turbo_kernel<8, 6, TW>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((attn_turbo_kernel<-1, -1, TW>), grid, block, 0, st, a);
+}
+
+}  // namespace oom
+
 extern "C" size_t oom_attn_decode_turbo_workspace_size(int heads, int kv_heads, int d, int kv_len) {
     if (heads < 1 || kv_heads < 1 || d < 1 || kv_len < 1 || heads % kv_heads) return 0;
-    return oom::turbo_ws(kv_heads, kv_len).total;
+    // every split of up to kv_len keys fits: blocks of 4 groups, at most TT_FILL over the KV heads
+    return oom::turbo_bytes(kv_heads, std::min((kv_len + 63) / 64, std::max(1, oom::TT_FILL / kv_heads)));
 }
 
 extern "C" int oom_attn_decode_turbo(const float* q, const uint8_t* k, const uint8_t* v, int k_bits, int v_bits,
@@ -1092,8 +1139,9 @@ extern "C" int oom_attn_decode_turbo(const float* q, const uint8_t* k, const uin
     OOM_REQUIRE((int64_t)kv_len * kv_heads * kv_row_bytes(d, std::max(k_bits, v_bits)) < TQ_OOB,
                 "oom_attn_decode_turbo: cache too large (rows of one cache under 1.75 GiB)");
     OOM_REQUIRE(q && k && v && mask && out && (k_bits == 0 || levels), "oom_attn_decode_turbo: null buffer");
-    const TurboWs w = turbo_ws(kv_heads, kv_len);
-    if (!ws || ws_bytes < w.total)
+    TurboSplit sp = turbo_split(kv_len, kv_heads, k_bits == 0);
+    if (ws_bytes < turbo_bytes(kv_heads, sp.blocks)) sp = turbo_split_least(kv_len, kv_heads);
+    if (!ws || ws_bytes < turbo_bytes(kv_heads, sp.blocks))
         return fail(OOM_ERR_WORKSPACE,
                     "oom_attn_decode_turbo: workspace smaller than oom_attn_decode_turbo_workspace_size()");
     OOM_REQUIRE(aligned(ws, 256), "oom_attn_decode_turbo: workspace must be 256-byte aligned");
@@ -1105,19 +1153,17 @@ extern "C" int oom_attn_decode_turbo(const float* q, const uint8_t* k, const uin
     a.v = v;
     a.mask = mask;
     a.levels = levels;
-    a.part = reinterpret_cast<float*>(base + w.part);
-    a.ml = reinterpret_cast<float*>(base + w.ml);
+    a.part = reinterpret_cast<float*>(base);
+    a.ml = reinterpret_cast<float*>(base + turbo_ml(kv_heads, sp.blocks));
     a.out = out;
     a.Hkv = kv_heads;
     a.kv_len = kv_len;
-    a.nblk = w.nblk;
+    a.nblk = sp.blocks;
     a.kb = k_bits;
     a.vb = v_bits;
     a.scale = scale;
-    const dim3 grid((unsigned)w.nblk, (unsigned)kv_heads), block(TT_WAVES * 64);
-    if (k_bits == 0) hipLaunchKernelGGL((attn_turbo_kernel<0, 0>), grid, block, 0, st, a);
-    else if (k_bits == 8 && v_bits == 6) hipLaunchKernelGGL((attn_turbo_kernel<8, 6>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((attn_turbo_kernel<-1, -1>), grid, block, 0, st, a);
+    if (sp.waves == 4) launch_turbo<4>(a, st);
+    else launch_turbo<8>(a, st);
     if (int rc = launched("oom_attn_decode_turbo")) return rc;
     if (k_bits == 0) hipLaunchKernelGGL(attn_turbo_combine_kernel<false>, dim3((unsigned)heads), dim3(TC_THREADS), 0, st, a);
     else hipLaunchKernelGGL(attn_turbo_combine_kernel<true>, dim3((unsigned)heads), dim3(TC_THREADS), 0, st, a);

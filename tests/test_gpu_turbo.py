@@ -175,3 +175,50 @@ def test_decode_turbo_rejects_bad_shapes(hip):
     q24 = torch.zeros((24, 256), dtype=torch.float32, device="cuda")
     with pytest.raises(hip.OomError, match="both 0"):
         hip.attn_decode_turbo(q24, k, k, 8, 0, lv, m, 2, 4, 0.1, torch.zeros_like(q24), ws)
+
+
+@pytest.mark.parametrize("Hkv,kv_len,kb,vb,mk", [
+    (1, 16, 8, 6, "all"), (2, 65, 8, 6, "all"),        # one block; two blocks of 4 waves, the last nearly empty
+    (2, 8192, 8, 6, "qsa"), (2, 8193, 4, 3, "all"),    # 256 blocks of 4 waves; past them, blocks of 8
+    (2, 8193, 0, 0, "qsa"), (4, 8193, 0, 0, "all"),    # fp32 rows: 4 waves of two groups; past them, blocks of 8
+    (3, 10901, 4, 4, "qsa"),                           # 8 waves, one group a wave, an uneven share a KV head
+    (4, 16400, 8, 6, "all"),                           # 8 waves of more than one group
+])
+def test_decode_turbo_splits(hip, levels, Hkv, kv_len, kb, vb, mk):
+    """Every way a KV head's keys are dealt, at the sizes where the rule changes, against the
+    oracle (the file's 2e-5 of scale) and against the split of the smallest workspace (the same
+    sums in another order and other reference maxima: fp32 rounding of ~2^-24 a term through
+    __expf's 2^-21, so 4e-6 of scale)."""
+    import torch
+
+    print(f"case: turbo split Hkv={Hkv} kv_len={kv_len} k{kb}v{vb} mask={mk}", flush=True)
+    D, H = 256, 12 * Hkv
+    rng = np.random.default_rng(kv_len + kb)
+    q = rng.standard_normal((H, D)).astype(np.float32)
+    mask = np.ones(kv_len, dtype=np.uint8) if mk == "all" else qsa_mask(kv_len, rng)
+    caches = []
+    for bits in (kb, vb):
+        c = torch.zeros(kv_len * Hkv * hip.kv_row_bytes(D, bits), dtype=torch.uint8, device="cuda")
+        hip.kv_append(torch.from_numpy(rng.standard_normal((kv_len, Hkv, D)).astype(np.float32)).cuda(), c, 0, bits,
+                      levels)
+        caches.append(c)
+    blocks = min(-(-kv_len // 256), max(1, 256 // Hkv))
+    least = (Hkv * blocks * 12 * 256 * 4 + 255) // 256 * 256 + (Hkv * blocks * 12 * 8 + 255) // 256 * 256
+    full = hip.attn_decode_turbo_workspace_size(H, Hkv, D, kv_len)
+    assert full >= least
+    outs = []
+    for size in (full, least):
+        ws = torch.zeros(size, dtype=torch.uint8, device="cuda")
+        out = torch.empty((H, D), dtype=torch.float32, device="cuda")
+        args = (torch.from_numpy(q).cuda(), *caches, kb, vb, levels, torch.from_numpy(mask).cuda(), Hkv, kv_len,
+                1.0 / 16.0, out)
+        hip.attn_decode_turbo(*args, ws)
+        outs.append(out.cpu().numpy())
+    with pytest.raises(hip.OomError, match="workspace"):
+        hip.attn_decode_turbo(*args, ws[:least - 256])
+    want = oracle.attn_decode_turbo(q, *(c.cpu().numpy() for c in caches), kb, vb, mask, H, Hkv, kv_len, 1.0 / 16.0)
+    mag = max(1.0, float(np.abs(want).max()))
+    assert np.abs(outs[0] - want).max() < 2e-5 * mag
+    assert np.abs(outs[0] - outs[1]).max() < 4e-6 * mag
+    sizes = [hip.attn_decode_turbo_workspace_size(H, Hkv, D, n) for n in range(1, 40000, 37)]
+    assert sizes == sorted(sizes)
