@@ -21,6 +21,9 @@
 // compiler's waits for the load ring stay exact. LDS rows are 40 bf16 (80 bytes), so
 // the 16 rows of an operand read fall in distinct bank groups. Grid (ceil(N / 128),
 // ceil(max_per_expert / 64), n_experts), as the reference's.
+#include <algorithm>
+
+#include "nvfp4_rows.hpp"
 #include "stream.hpp"
 
 namespace oom {
@@ -207,8 +210,9 @@ __global__ void __launch_bounds__(T4_THREADS, 2) moe_tiled_nvfp4_kernel(TiledArg
         }
 }
 
-// ---- wide tiles: all 640 rows of a projection tile over 64 assignments ---------------
+// ---- wide tiles: all 640 rows of a projection tile over 48 assignments ---------------
 //
+// For K past the few-row kernel's slices, or where rows_kernel_serves finds these the better.
 // The 128-row tiles above gather every activation row once per N tile, four times the
 // bytes of the weights they meet. Here a block of 8 waves takes 640 weight rows (wave w:
 // rows 80 w .. + 80, five 16-row N subtiles) x 64 assignments, so a gate or up projection
@@ -379,6 +383,161 @@ __global__ void __launch_bounds__(TW_THREADS) moe_tiled_nvfp4_wide_kernel(TiledA
         }
 }
 
+// ---- tiles of at most 16 assignments: weight rows streamed against registers ------------
+// (nvfp4_rows.hpp) One block a CU. The blocks count every expert's 16-row tiles, times the
+// batches of 128 weight rows a row group that a projection has, and each takes an equal run of
+// those units, so no CU waits for a last round of blocks: 511 experts' tiles and 14 second
+// ones as a block each took 180 us a projection of 640 x 2560, the equal runs 147. What bounds
+// it there: the decoding and the matrix cores of two waves a SIMD (184 vector instructions and
+// 30 MFMAs a 16-row subtile and slice, about 90 us) beside the stream (77 us at 6.1 TB/s).
+constexpr int TR_LIST = 1024;  // tiles a block can have
+
+template <int TERMS, int ST>
+__global__ void __launch_bounds__(64 * NR_WAVES) moe_tiled_nvfp4_rows_kernel(TiledArgs g, int n_experts, int max_n,
+                                                                            int batches, int ks_log) {
+    __shared__ RowsLds lds;
+    __shared__ int2 list[TR_LIST];
+    __shared__ int wtot[NR_WAVES];
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = 1 << ks_log, slice = wave & (ks - 1), group = wave >> ks_log, ngroups = NR_WAVES >> ks_log;
+    // ---- the block's share of the tiles' batches: tiles counted in expert order
+    const int per = (n_experts + 64 * NR_WAVES - 1) / (64 * NR_WAVES);
+    const int e0 = min(n_experts, tid * per), e1 = min(n_experts, e0 + per);
+    auto rows_of = [&](int e) { return min(max(g.off[e + 1] - g.off[e], 0), max_n); };
+    auto tiles_of = [&](int e) { return (rows_of(e) + NR_M - 1) / NR_M; };
+    int mine = 0;
+    for (int e = e0; e < e1; e++) mine += tiles_of(e);
+    int incl = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += v;
+    }
+    if (lane == 63) wtot[wave] = incl;
+    __syncthreads();
+    int total = 0, at = incl - mine;
+#pragma unroll
+    for (int w = 0; w < NR_WAVES; w++) {
+        if (w < wave) at += wtot[w];
+        total += wtot[w];
+    }
+    const int64_t units = (int64_t)total * batches;
+    const int u0 = (int)(units * blockIdx.x / gridDim.x), u1 = (int)(units * (blockIdx.x + 1) / gridDim.x);
+    if (u0 == u1) return;  // uniform over the block
+    const int t0 = u0 / batches, t1 = (u1 - 1) / batches;
+    for (int e = e0; e < e1; e++)
+        for (int z = 0, n = tiles_of(e); z < n; z++, at++)
+            if (at >= t0 && at <= t1) list[at - t0] = make_int2(e, z);
+    __syncthreads();
+    for (int u = u0; u < u1;) {
+        // batches first_b .. first_b + nb of one tile
+        const int2 tile = list[u / batches - t0];
+        const int e = __builtin_amdgcn_readfirstlane(tile.x), z = __builtin_amdgcn_readfirstlane(tile.y);
+        const int first_b = u % batches, nb = min(batches - first_b, u1 - u);
+        u += nb;
+        const int a0 = g.off[e] + NR_M * z, nt = min(NR_M, rows_of(e) - NR_M * z);
+        const int row0 = 16 * NR_BATCH * ngroups * first_b;  // the first weight row
+        const uint64_t rec = g.recs[e];
+        RowsW<ST> w;
+        w.init(lds, rec, g.w_off, g.s_off, g.N, g.K, row0 + 16 * NR_BATCH * group, lane, wave, slice, ks_log);
+        typename RowsW<ST>::Ld ld[4];
+        w.sload(0, true);
+#pragma unroll
+        for (int i = 0; i < 4; i++) w.load(ld[i], i, true);
+        // an operand row past the tile repeats its first one; its sums are not stored
+        const int a = a0 + (r < nt ? r : 0);
+        const float* xrow = g.x + (int64_t)(g.rows ? g.rows[a] : a) * g.K;
+        const int kq = 32 * ST * slice + 8 * ST * q;
+        RowsX<TERMS, ST> x;
+        if (g.K == 32 * ST * ks) x.template load<false>(xrow, kq, g.K);
+        else x.template load<true>(xrow, kq, g.K);
+        // (a buffer load: through a generic pointer it is a flat load, and with one pending every
+        // wait for a load waits for all of them)
+        const float s2 = ldf(uniform_rsrc(rec + 4ull * (unsigned)g.s2_idx, 4), 0);
+        w.sput(lane);
+        __syncthreads();
+        for (int b = 0; b < nb; b++) {
+            const int sub = NR_BATCH * ngroups * b;  // subtiles before the batch, in the group's count
+            w.sload(sub + NR_BATCH * ngroups, b + 1 < nb);
+            // a subtile's operands are staged while the one before is on the matrix cores
+            typename RowsW<ST>::Op op[2];
+            w.stage(ld[0], 0, op[0]);
+#pragma unroll
+            for (int i = 0; i < NR_BATCH; i++) {
+                if (i < NR_BATCH - 4) w.load(ld[i & 3], sub + i + 4, true);
+                else w.load(ld[i & 3], sub + NR_BATCH * ngroups + i + 4 - NR_BATCH, b + 1 < nb);
+                if (i + 1 < NR_BATCH) w.stage(ld[(i + 1) & 3], i + 1, op[(i + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                lds.red[wave][i][lane] = w.dot(op[i & 1], x);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __syncthreads();
+            w.sput(lane);
+            // the batch's ngroups x NR_BATCH subtiles, ngroups of them a wave
+            const auto put = [&](int gs, n4f4 y) {
+                const int row = row0 + 16 * (sub + gs) + r;
+                if (row < g.N)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        if (4 * q + j < nt) g.y[(int64_t)(a0 + 4 * q + j) * g.N + row] = y[j] * s2;
+            };
+            if (ks == 8) rows_meet<3>(lds, wave, lane, put);
+            else if (ks == 4) rows_meet<2>(lds, wave, lane, put);
+            else if (ks == 2) rows_meet<1>(lds, wave, lane, put);
+            else rows_meet<0>(lds, wave, lane, put);
+            __syncthreads();
+        }
+    }
+}
+
+static int rows_batches(int64_t N, const RowsSplit& sp) {
+    return (int)cdiv(N, 16 * NR_BATCH * (NR_WAVES >> sp.ks_log));
+}
+
+// Where the rows kernel is the better one: K in whole scale groups a lane and at most 8 slices
+// of 10 steps, and either slices and batches that K and N fill (five sixths at least) or tiles
+// of so few rows that the stream counts and not the steps. Us a call of gate, up, SwiGLU, down
+// and combine at 2560 / 640, exact, rows kernel and tiles: 512 experts top-10, 60 tokens 287
+// and 601, 250 398 and 698, 500 451 and 722, 900 664 and 761, 1050 766 and 782, 1400 924 and
+// 1224, 2048 1218 and 1472; 64 experts, 300 tokens 228 and 296, 1200 612 and 626. At 1600 / 448
+// (slices 78 % and 88 % full) 128 experts top-4, 600 tokens 151 and 185, but 64 experts top-10,
+// 1200 tokens (190 rows an expert) 398 and 327. The tiles also keep the steps of many experts
+// whose 41 to 48 rows at most are one 48-row tile where the rows kernel decodes twice or more
+// (512 experts, 1200 tokens: 815 and 786; with 128 experts 264 and 299).
+static bool rows_kernel_serves(int64_t N, int64_t K, int64_t w_off, int64_t s_off, int64_t n_experts, int64_t max_n,
+                               bool exact) {
+    if (K % 64 != 0 || K > NR_MAXK || w_off % 4 != 0 || s_off % 4 != 0) return false;
+    const RowsSplit sp = rows_split(K);
+    if (n_experts * cdiv(max_n, NR_M) * rows_batches(N, sp) > INT32_MAX) return false;
+    if (exact && K % TW_BK == 0 && n_experts >= 384 && max_n > 40 && max_n <= TW_BM) return false;
+    const int64_t rows = (int64_t)16 * NR_BATCH * (NR_WAVES >> sp.ks_log) * rows_batches(N, sp);
+    return 6 * K * N >= 5 * ((int64_t)32 * sp.st << sp.ks_log) * rows || max_n <= 48;
+}
+
+template <int TERMS>
+static void launch_tiled_rows(const TiledArgs& a, int n_experts, int max_per_expert, hipStream_t st) {
+    const RowsSplit sp = rows_split(a.K);
+    const int batches = rows_batches(a.N, sp);
+    const int64_t most = (int64_t)n_experts * cdiv(max_per_expert, NR_M);  // tiles
+    const dim3 grid((unsigned)std::max(std::min<int64_t>(256, most * batches), cdiv(most, TR_LIST - 2)));
+    const dim3 block(64 * NR_WAVES);
+    switch (sp.st) {
+        case 6:
+            hipLaunchKernelGGL((moe_tiled_nvfp4_rows_kernel<TERMS, 6>), grid, block, 0, st, a, n_experts,
+                               max_per_expert, batches, sp.ks_log);
+            break;
+        case 8:
+            hipLaunchKernelGGL((moe_tiled_nvfp4_rows_kernel<TERMS, 8>), grid, block, 0, st, a, n_experts,
+                               max_per_expert, batches, sp.ks_log);
+            break;
+        default:
+            hipLaunchKernelGGL((moe_tiled_nvfp4_rows_kernel<TERMS, 10>), grid, block, 0, st, a, n_experts,
+                               max_per_expert, batches, sp.ks_log);
+            break;
+    }
+}
+
 __global__ void __launch_bounds__(256) moe_swiglu_kernel(const float* __restrict__ gt, const float* __restrict__ up,
                                                          float* __restrict__ h, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -403,6 +562,12 @@ extern "C" int oom_moe_tiled_nvfp4(const uint64_t* recs, const int32_t* off, con
     OOM_REQUIRE(recs && off && x && y, "oom_moe_tiled_nvfp4: null buffer");
     OOM_REQUIRE(aligned(x, 16), "oom_moe_tiled_nvfp4: x must be 16-byte aligned");
     TiledArgs a{recs, off, rows, x, y, n, k, w_off, s_off, s2_idx};
+    if (rows_kernel_serves(n, k, w_off, s_off, n_experts, max_per_expert,
+                           precision == OOM_EXPERT_EXACT)) {
+        if (precision == OOM_EXPERT_EXACT) launch_tiled_rows<3>(a, n_experts, max_per_expert, as_stream(stream));
+        else launch_tiled_rows<1>(a, n_experts, max_per_expert, as_stream(stream));
+        return launched("oom_moe_tiled_nvfp4");
+    }
     if (k % TW_BK == 0 && w_off % 16 == 0 && s_off % 2 == 0) {
         // 640-row tiles, weights straight into registers (records' parts are 16-byte aligned
         // in the released layout)

@@ -91,3 +91,39 @@ def test_swiglu_range(hip):
     want = (g.astype(np.float64) / (1.0 + np.exp(-g.astype(np.float64)))) * u
     assert np.all(got[:13] == -9.0) and np.all(got[9001:] == -9.0)
     np.testing.assert_allclose(got[13:9001], want[13:9001], rtol=4e-7, atol=1e-30)
+
+
+@pytest.mark.parametrize("n,k,counts", [
+    (40, 64, [1, 16, 17]),              # one slice, fewer columns than its steps; one part of a batch
+    (130, 192, [15, 0, 33]),            # an empty expert, a second row group's first rows
+    (640, 320, [48, 2]),                # one slice filled
+    (300, 384, [16, 5]),                # two slices of 6 steps
+    (520, 1088, [7, 31]),               # four slices, the last one part filled
+    (1100, 2496, [3, 18]),              # eight slices of 10 steps, the last one part filled
+    (96, 1536, [16] * 20),              # eight slices of 6 steps, more tiles than experts' share of a block
+    (16, 128, [1, 0, 2] * 300),         # more experts than threads that count them
+    (64, 256, [200]),                   # one expert, many tiles
+    (200, 2688, [3, 50]),               # past 8 slices of 10 steps: the 48-row tiles
+])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_tiled_rows_kernel(hip, n, k, counts, precision):
+    """The few-row kernel's slices, row groups, tiles and shares at their edges (the file's f64
+    bar), with the rows in any order and without a row list."""
+    import torch
+
+    print(f"case: tiled rows n={n} k={k} experts={len(counts)} precision={precision}", flush=True)
+    recs, x, off, rows = case(n, k, counts, 5 + n + k)
+    A = int(off[-1])
+    buf = torch.from_numpy(np.stack(recs.recs)).cuda()
+    addrs = torch.tensor([buf.data_ptr() + e * recs.stride for e in range(len(counts))], dtype=torch.int64,
+                         device="cuda")
+    for row_list in (True, False):
+        xs = x if row_list else x[rows]
+        y = torch.full((A + 3, n), float("nan"), dtype=torch.float32, device="cuda")
+        hip.moe_tiled_nvfp4(addrs, torch.from_numpy(off).cuda(), torch.from_numpy(rows).cuda() if row_list else None,
+                            len(counts), max(counts), torch.from_numpy(np.ascontiguousarray(xs)).cuda(), y, n, k,
+                            recs.w_off, recs.s_off, 0, precision)
+        got = y.cpu().numpy()
+        want, mag = f64_eval(recs, x, off, rows, precision == 0)
+        assert np.isnan(got[A:]).all(), "rows past the assignments were written"
+        assert (np.abs(got[:A] - want) / mag).max() < 2e-6
