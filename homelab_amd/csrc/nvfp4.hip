@@ -91,18 +91,18 @@ __device__ __forceinline__ uint32_t ldb(__amdgpu_buffer_rsrc_t r, int off) {
 __device__ __forceinline__ float e4m3_byte(uint32_t b) { return __builtin_amdgcn_cvt_f32_fp8((int)b, 0); }
 
 // Stages rows row_of(t) (t < nb) of src (width K, element type DT) into LDS in the lane
-// order above; zeros past K and for t >= nb. 256 threads take part, thread ti of them.
-template <int DT, typename RowOf>
+// order above; zeros past K and for t >= nb. NT threads take part, thread ti of them.
+template <int DT, int NT = 256, typename RowOf>
 __device__ __forceinline__ void stage4(float4* xs4, const void* src, int K, int CH, int nb, RowOf row_of,
                                        int ti = (int)threadIdx.x) {
     constexpr int EPL = DT == OOM_BF16 ? 8 : 4;  // elements per 16-byte load
     constexpr int ES = DT == OOM_BF16 ? 2 : 4;
     const int span = CH * 1024, nvec = N4_TB * span / EPL;
-    for (int base = 0; base < nvec; base += 256 * 4) {
+    for (int base = 0; base < nvec; base += NT * 4) {
         uint4 v[4];
 #pragma unroll
         for (int n = 0; n < 4; n++) {
-            const int i = base + ti + 256 * n;
+            const int i = base + ti + NT * n;
             const int t = i * EPL / span, kk = i * EPL - t * span;
             const bool ok = i < nvec && t < nb && kk < K;
             v[n] = ok ? *reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(src) +
@@ -111,7 +111,7 @@ __device__ __forceinline__ void stage4(float4* xs4, const void* src, int K, int 
         }
 #pragma unroll
         for (int n = 0; n < 4; n++) {
-            const int i = base + ti + 256 * n;
+            const int i = base + ti + NT * n;
             if (i >= nvec) break;
             const int t = i * EPL / span, kk = i * EPL - t * span;
             const int c = kk >> 10, l = (kk & 1023) >> 5, j = kk & 31;
@@ -517,6 +517,87 @@ __device__ __forceinline__ void dn4_compute(const Dn4W& w, const float4* xs4, co
     }
 }
 
+// ---- a few tokens: the routed experts' rows streamed once by free-running waves --------------
+// The staged gate/up above is a chain per block (plan entries, activations into LDS, a round
+// of weights, the sums, the end), two blocks a CU: at 8 tokens, 512 experts top-10, 2560 / 640,
+// 51.7 us for 147 MB. Here a block a CU stages every token's x once, and its waves then take
+// items with no block sync between them, the next item's loads in flight behind the current
+// one's sums: 40 us there, bound by the conversions and sums of the assignments. The
+// arithmetic is gu4_math's, so every output has the staged kernel's bits. Down stays staged:
+// the same form of it re-reads an expert's h per wave and took 39 us against 30.
+constexpr int N4S_WAVES = 8;
+constexpr int N4S_AMAX = 512;               // assignments of a step (and so routed experts)
+constexpr size_t N4S_XMAX = 144 * 1024;     // of LDS for the tokens' x, beside the plan's 12 KiB
+
+// The step's plan as the waves read it.
+struct Plan4Lds {
+    uint64_t recs[N4S_AMAX];
+    float s2[N4S_AMAX][2];
+    int off[N4S_AMAX + 1];
+    int tok[N4S_AMAX];
+};
+
+template <int XDT, int CS>
+__global__ void __launch_bounds__(64 * N4S_WAVES) moe_gate_up_nvfp4_step_kernel(
+    const uint64_t* __restrict__ recs, const int32_t* __restrict__ off, const int32_t* __restrict__ assign_tok,
+    const void* __restrict__ x, int T, float* __restrict__ h, Rec4 g, const int32_t* __restrict__ n_e_dev) {
+    extern __shared__ float4 xs4[];
+    __shared__ Plan4Lds pl;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int H = g.H, I = g.I, CH = (H + 1023) >> 10;
+    const int ipe = (I + 2 * N4_GP - 1) / (2 * N4_GP), NG = *n_e_dev * ipe, NW = gridDim.x * N4S_WAVES;
+    // items it0, it0 + NW, ...: neighbouring items on different CUs
+    int it = wave * gridDim.x + blockIdx.x;
+    const auto rsrc_of = [&](int item, uint64_t rec) { return uniform_rsrc(rec, item < NG ? g.bytes : 0); };
+    Gu4Ld<CS> ta, tb;
+    {
+        const int e = min(it, NG - 1) / ipe;
+        gu4_load<CS>(g, rsrc_of(it, recs[e]), (it - e * ipe) * 2 * N4_GP, lane, 0, ta);
+    }
+    // the plan and every token's x into LDS (stage4's lane order)
+    const int n_e = *n_e_dev;
+    if ((int)threadIdx.x < n_e) {
+        const int e = threadIdx.x;
+        const uint64_t rec = recs[e];
+        pl.recs[e] = rec;
+        pl.off[e] = off[e];
+        if (e == n_e - 1) pl.off[n_e] = off[n_e];
+        pl.s2[e][0] = *reinterpret_cast<const __attribute__((address_space(1))) float*>(rec + g.s2g);
+        pl.s2[e][1] = *reinterpret_cast<const __attribute__((address_space(1))) float*>(rec + g.s2u);
+    }
+    const int A = off[n_e];
+    if ((int)threadIdx.x < A) pl.tok[threadIdx.x] = assign_tok[threadIdx.x];
+    for (int t = 0; t < T; t += N4_TB)
+        stage4<XDT, 64 * N4S_WAVES>(xs4 + (size_t)t * CH * 256, x, H, CH, min(N4_TB, T - t), [&](int i) { return t + i; });
+    __syncthreads();
+    const auto sums = [&](int item, const Gu4Ld<CS>& t) {
+        const int e = __builtin_amdgcn_readfirstlane(item / ipe), j0 = (item - e * ipe) * 2 * N4_GP;
+        const int a0 = __builtin_amdgcn_readfirstlane(pl.off[e]), a1 = __builtin_amdgcn_readfirstlane(pl.off[e + 1]);
+        const float s2g = pl.s2[e][0], s2u = pl.s2[e][1];
+        for (int a = a0; a < a1; a++) {
+            const int tok = __builtin_amdgcn_readfirstlane(pl.tok[a]);
+            float acc[2 * N4_GP];
+#pragma unroll
+            for (int i = 0; i < 2 * N4_GP; i++) acc[i] = 0.0f;
+            gu4_math<1, CS>(xs4 + (size_t)tok * CH * 256, g, s2g, s2u, lane, 0, t, acc);
+            gu4_put<1>(acc, I, j0, lane, 1, [&](int, int j, float v) { h[(size_t)a * I + j] = v; });
+        }
+    };
+    const auto load = [&](int item, Gu4Ld<CS>& t) {
+        const int e = __builtin_amdgcn_readfirstlane(min(item, NG - 1) / ipe);
+        gu4_load<CS>(g, rsrc_of(item, pl.recs[e]), (item - e * ipe) * 2 * N4_GP, lane, 0, t);
+    };
+    while (it < NG) {
+        load(it + NW, tb);
+        sums(it, ta);
+        it += NW;
+        if (it >= NG) break;
+        load(it + NW, ta);
+        sums(it, tb);
+        it += NW;
+    }
+}
+
 template <int XDT, int EQ, int ODT>
 __global__ void __launch_bounds__(256) moe_decode_nvfp4_1_kernel(Fused4Args a) {
     const uint32_t bbase = grid_barrier_base(a.bar);
@@ -884,6 +965,49 @@ static int launch_gate_up4(const uint64_t* recs, const int32_t* off, const int32
     return launched("oom_moe_gate_up_nvfp4");
 }
 
+// A step whose tokens' x fits LDS beside the plan, with rows enough (the most that its
+// assignments can reach) to pay for staging all of x in every block. The whole step, staged
+// against this: 64 experts of 1040 / 272 (18 M) 35.6 and 38.3 us, 8 of 1024 / 256 (2 M) 20.0
+// and 20.9; 20 of 2560 / 640 (33 M) 40.4 and 40.0, 80 (131 M) 97 and 86, 144 of 2560 / 1536
+// (566 M) 113 and 95.
+constexpr int64_t N4S_MIN_ROWS = 24ll << 20;  // experts x hidden x inter
+static size_t gate_up_step_lds(int T, const OomNvfp4Record& g) {
+    return (size_t)((T + 1) / 2 * 2) * cdiv(g.hidden, 1024) * 4096;  // staged two rows at a time
+}
+static bool gate_up_step_ok(int T, int A, int grid_e, const OomNvfp4Record& g) {
+    return A <= N4S_AMAX && gate_up_step_lds(T, g) <= N4S_XMAX && grid_e * g.hidden * g.inter >= N4S_MIN_ROWS;
+}
+
+template <int XDT, int CS>
+static int launch_gate_up_step_t(const uint64_t* recs, const PlanView& pv, const void* x, int T, float* h,
+                                 const OomNvfp4Record& geo, hipStream_t st) {
+    const size_t lds = gate_up_step_lds(T, geo);
+    static thread_local int raised_dev = -1;  // the device whose limit on dynamic LDS was raised
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    if (dev != raised_dev) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gate_up_nvfp4_step_kernel<XDT, CS>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)N4S_XMAX) != hipSuccess)
+            return fail(OOM_ERR_LAUNCH, "oom_moe_decode_nvfp4: the device refused the step's LDS");
+        raised_dev = dev;
+    }
+    hipLaunchKernelGGL((moe_gate_up_nvfp4_step_kernel<XDT, CS>), dim3(256), dim3(64 * N4S_WAVES), lds, st, recs, pv.off(),
+                       pv.assign_tok(), x, T, h, rec4_of(geo), pv.n_e());
+    return launched("moe_gate_up_nvfp4");
+}
+
+static int launch_gate_up_step(const uint64_t* recs, const PlanView& pv, const void* x, int xdt, int T, float* h,
+                               const OomNvfp4Record& geo, hipStream_t st) {
+    const int ch = (int)cdiv(geo.hidden, 1024);
+#define N4S_CASE(C)                                                                                    \
+    return xdt == OOM_BF16 ? launch_gate_up_step_t<OOM_BF16, C>(recs, pv, x, T, h, geo, st)             \
+                           : launch_gate_up_step_t<OOM_F32, C>(recs, pv, x, T, h, geo, st);
+    if (ch <= 2) { N4S_CASE(2) }
+    if (ch == 3) { N4S_CASE(3) }
+    N4S_CASE(4)
+#undef N4S_CASE
+}
+
 static int launch_down4(const uint64_t* recs, const int32_t* off, int grid_e, const float* h, float* y,
                         const OomNvfp4Record& geo, const int32_t* n_e_dev, hipStream_t st) {
     const Rec4 g = rec4_of(geo);
@@ -981,7 +1105,11 @@ extern "C" int oom_moe_decode_nvfp4(const float* logits, const void* x, int x_dt
     if (int rc = oom_router_topk(logits, ids, weights, T, E, k, stream)) return rc;
     if (int rc = oom_moe_plan(ids, T, E, k, all_recs, plan, recs, stream)) return rc;
     const int grid_e = std::min(E, A);
-    if (int rc = launch_gate_up4(recs, pv.off(), pv.assign_tok(), grid_e, x, x_dtype, h, *geo, pv.n_e(), st)) return rc;
+    if (gate_up_step_ok(T, A, grid_e, *geo)) {
+        if (int rc = launch_gate_up_step(recs, pv, x, x_dtype, T, h, *geo, st)) return rc;
+    } else if (int rc = launch_gate_up4(recs, pv.off(), pv.assign_tok(), grid_e, x, x_dtype, h, *geo, pv.n_e(), st)) {
+        return rc;
+    }
     if (int rc = launch_down4(recs, pv.off(), grid_e, h, y, *geo, pv.n_e(), st)) return rc;
     return launch_combine(y, pv.slot_assign(), weights, out, out_dtype, T, (int)geo->hidden, k, st);
 }

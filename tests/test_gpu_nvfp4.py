@@ -245,3 +245,56 @@ def _one_launch_check(hip, E, k, H, I, xf32, seed, logits):
     bad = ~np.isclose(got, want_or, rtol=RTOL, atol=ATOL)
     assert not bad.any(), f"{bad.sum()} of {bad.size} outside; worst {np.abs(got - want_or)[bad].max():.3e}"
     assert hip.status() == hip.OK, "a wait of the one-launch kernel gave up"
+
+
+@pytest.mark.parametrize("T,E,k,H,I,levels,xf32", [
+    (2, 64, 8, 4096, 1536, 8.0, True),     # four chunks a row; two tokens staged
+    (9, 64, 8, 4096, 768, 8.0, True),      # odd token count whose padded x overflows LDS: the staged launch
+    (8, 512, 10, 2560, 640, 8.0, False),   # three chunks
+    (13, 128, 10, 2064, 528, 2.0, True),   # odd count; rows past a whole item; widths ending inside a chunk
+    (32, 128, 16, 1008, 304, 2.0, False),  # A = 512, the plan's most, experts with many tokens
+    (33, 128, 16, 1008, 304, 2.0, False),  # A = 528: the staged launch
+    (7, 256, 4, 2048, 1552, 0.0, True),    # all logits equal: every token on the same four experts
+])
+def test_decode_nvfp4_step_matches_stages(hip, T, E, k, H, I, levels, xf32):
+    """Several tokens: the step's gate/up stages all of x per block and free-runs its waves
+    where x fits LDS. Its sums are the staged launch's in the staged order, so the f32 output
+    equals, bit for bit, the staged launches' over the same routing. Four records serve all
+    experts (record e % 4): only the arithmetic is compared here."""
+    import torch
+
+    print(f"case: nvfp4 step T={T} E={E} k={k} H={H} I={I} x={'f32' if xf32 else 'bf16'}", flush=True)
+    seed = 1200 + T + E + H
+    geo, hgeo = oracle.nvfp4_geometry(H, I), hip.nvfp4_geometry(H, I)
+    z = np.random.default_rng(seed).standard_normal((T, E))
+    logits = (np.round(z * levels) / levels if levels else np.zeros_like(z)).astype(np.float32)
+    buf, four = _upload(synth.nvfp4_records(geo, seed, 4))
+    addrs = four[torch.arange(E, device="cuda") % 4].contiguous()
+    xb = synth.activations_bf16(seed, T, H)
+    xd = _dev(oracle.bf16_to_f32(xb)) if xf32 else _bf16(xb)
+    ld = _dev(logits)
+    ids_s = torch.empty((T, k), dtype=torch.int32, device="cuda")
+    w_s = torch.empty((T, k), dtype=torch.float32, device="cuda")
+    hip.router_topk(ld, ids_s, w_s, k)
+    torch.cuda.synchronize()
+    experts, off, tok, slot = oracle.moe_plan(ids_s.cpu().numpy(), E)
+    n_e = len(experts)
+    recs_s = addrs[torch.from_numpy(np.asarray(experts, dtype=np.int64)).cuda()]
+    offd, tokd = _dev(np.asarray(off, dtype=np.int32)), _dev(np.asarray(tok, dtype=np.int32))
+    h = torch.empty((T * k, I), dtype=torch.float32, device="cuda")
+    y = torch.empty((T * k, H), dtype=torch.float32, device="cuda")
+    hip.moe_gate_up_nvfp4(recs_s, offd, tokd, n_e, xd, h, hgeo)
+    hip.moe_down_nvfp4(recs_s, offd, n_e, h, y, hgeo)
+    want = torch.empty((T, H), dtype=torch.float32, device="cuda")
+    hip.moe_combine_slots(y, _dev(np.asarray(slot, dtype=np.int32).reshape(T, k)), w_s, want)
+    torch.cuda.synchronize()
+    ws = torch.zeros(hip.moe_decode_nvfp4_workspace_size(T, E, k, hgeo), dtype=torch.uint8, device="cuda")
+    ids = torch.empty((T, k), dtype=torch.int32, device="cuda")
+    w = torch.empty((T, k), dtype=torch.float32, device="cuda")
+    for rep in range(2):
+        out = torch.full((T, H), float("nan"), dtype=torch.float32, device="cuda")
+        hip.moe_decode_nvfp4(ld, xd, addrs, k, hgeo, ids, w, out, ws)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(ids.cpu().numpy(), ids_s.cpu().numpy(), err_msg=f"rep {rep}")
+        diff = np.flatnonzero(out.cpu().numpy().view(np.uint32).ravel() != want.cpu().numpy().view(np.uint32).ravel())
+        assert diff.size == 0, f"rep {rep}: {diff.size} of {T * H} differ, first at {diff[:4]}"
