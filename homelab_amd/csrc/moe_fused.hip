@@ -623,7 +623,7 @@ __global__ void __launch_bounds__(TG == 1 ? 64 * FW1 : 64 * FW) moe_decode_fused
     // stores wait for their loads) and the activations load while the router runs
     float lv0[EQ];
     if constexpr (TG == 1) {
-        if (T == 1 && wave == 0) route_logits<EQ>(a.logits, E, lane, lv0);
+        if (wave == 0) route_logits<EQ>(a.logits, E, lane, lv0);
     }
     constexpr int RT0 = TG == 1 ? 64 : 0;  // first thread of the record-table copy
     static_assert(TG != 1 || 64 * FW1 >= 64 + F_EMAX + 1, "the other waves hold the record table");
@@ -658,7 +658,7 @@ __global__ void __launch_bounds__(TG == 1 ? 64 * FW1 : 64 * FW) moe_decode_fused
         }
     }
     // ---- routing and plan: slots sorted by (expert, slot), experts in id order ----
-    if (T == 1) {
+    if constexpr (TG == 1) {
         // one token: wave 0 routes it and plans in place, one block-wide sync
         if (wave == 0) {
             // picks and plan in one pass (ballot radix selection); with one token the

@@ -299,3 +299,36 @@ def test_fused_decode_full_size(hip, T, E, k, zipf, H, I):
     torch.cuda.synchronize()
     f64 = synth.f64_moe((want_ids, want_w), x, recs, geo)
     assert np.abs(out32.cpu().numpy() - f64).max() <= 2e-5 * np.abs(f64).max()
+
+
+@pytest.mark.parametrize("T,E,k,H,I,xf32", [
+    (1, 16, 9, 256, 128, False),     # one token, more experts than the one-token kernel's waves
+    (1, 64, 12, 512, 256, True),
+    (1, 256, 32, 1040, 272, False),  # the most picks; widths ending inside a chunk
+])
+def test_fused_decode_general(hip, T, E, k, H, I, xf32):
+    """The one-launch kernel for what the one-token and the MFMA batch kernels leave: one
+    token with more than 8 experts, f32 activations, more than 16 tokens. Ids and weights
+    as the oracle's; f32 output within 2e-5 of scale of the float64 evaluation, twice on
+    one workspace."""
+    import torch
+
+    print(f"case: fused general T={T} E={E} k={k} H={H} I={I} x={'f32' if xf32 else 'bf16'}", flush=True)
+    geo, logits, recs, xb = decode_case(T, E, k, None, 1500 + T + E, H, I)
+    x = oracle.bf16_to_f32(xb)
+    want_ids, want_w = oracle.router_topk(logits, k)
+    hgeo = hip.record_geometry(geo.hidden, geo.inter)
+    buf, addrs = upload_records(recs)
+    ws = torch.zeros(hip.moe_decode_fp8_workspace_size(T, E, k, hgeo), dtype=torch.uint8, device="cuda")
+    ids = torch.empty((T, k), dtype=torch.int32, device="cuda")
+    w = torch.empty((T, k), dtype=torch.float32, device="cuda")
+    ld, xd = dev(logits), dev(x) if xf32 else bf16_dev(xb)
+    f64 = synth.f64_moe((want_ids, want_w), x, recs, geo)
+    for rep in range(2):
+        out = torch.full((T, H), float("nan"), dtype=torch.float32, device="cuda")
+        hip.moe_decode_fp8(ld, xd, addrs, k, hgeo, ids, w, out, ws)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(ids.cpu().numpy(), want_ids, err_msg=f"rep {rep}")
+        np.testing.assert_allclose(w.cpu().numpy(), want_w, rtol=2e-6, err_msg=f"rep {rep}")
+        err = np.abs(out.cpu().numpy() - f64).max()
+        assert err <= 2e-5 * np.abs(f64).max(), f"rep {rep}: max err {err:.3e} vs scale {np.abs(f64).max():.3e}"
