@@ -41,7 +41,7 @@ namespace oom {
 constexpr int FW = 4;        // waves per block (more than one token)
 constexpr int FW1 = 8;       // waves per block with one token: one expert slot each
 constexpr int FD1_NP = 8;    // row pairs of a one-token down tile (16 rows)
-constexpr int FG_R = 2;      // gate (and up) rows per gate/up item
+constexpr int FG_R = 2;      // gate (and up) rows per gate/up item, several tokens
 constexpr int FD_R = 8;      // output rows per down item
 constexpr int F_AMAX = 512;  // assignments (T * k) per step
 constexpr int F_EMAX = 256;  // experts (register router; larger E takes the multi-launch path)
@@ -75,31 +75,6 @@ struct FusedArgs {
 #endif
 };
 
-// 16 consecutive activations of row `row` starting at column `col`, as fp32.
-template <int XDT>
-__device__ __forceinline__ void load16(const void* base, size_t off, float* v) {
-    if constexpr (XDT == OOM_BF16) {
-        const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(base) + off);
-        uint4 a = p[0], b = p[1];
-        uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            v[2 * i] = __uint_as_float(w[i] << 16);
-            v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-        }
-    } else {
-        const float4* p = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(base) + off);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float4 a = p[i];
-            v[4 * i] = a.x;
-            v[4 * i + 1] = a.y;
-            v[4 * i + 2] = a.z;
-            v[4 * i + 3] = a.w;
-        }
-    }
-}
-
 struct PlanLds {
     uint64_t recs[F_EMAX + 1];  // all_recs, read once per block (+ the shared expert's record)
     uint64_t keys[FW1];     // one-token routing scratch (route_select)
@@ -115,117 +90,220 @@ struct PlanLds {
     float w[F_AMAX];
 };
 
-template <int TG, int XDT>
-__device__ __forceinline__ void gate_up_item(const FusedArgs& a, const PlanLds& pl, int i, int tile, int lane) {
-    const int H = (int)a.H, I = (int)a.I;
-    const int CH = (H + 1023) >> 10, nkb = (H + 127) >> 7;
-    const uint8_t* rec = reinterpret_cast<const uint8_t*>(pl.recs[pl.experts[i]]);
-    const int j0 = tile * FG_R;
-    uint4 wg[FG_R][4], wu[FG_R][4];
+// A record's parts through one buffer resource; an empty resource (bytes 0) reads zeros.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rec_rsrc(const PlanLds& pl, int i, int bytes) {
+    const uint64_t r = pl.recs[pl.experts[i]];
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)r), hi = __builtin_amdgcn_readfirstlane((uint32_t)(r >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), (short)0, bytes,
+                                             BUF_FLAGS);
+}
+
+// ---- several tokens, or one with more than FW1 experts ------------------------------------
+// Bound by the rows' stream and, as tokens per expert grow, by the conversions and sums. A
+// wave's next item (gate/up or down) loads behind the current one's sums; an expert's first
+// token (the only one of most, at a few tokens) takes a pass of its own, its activations
+// loaded in one round ahead of the next item's rows, and the others go two a pass (four: 161
+// against 151 us at 16 tokens of the case below, and spills with f32 rows of 4096). All of a
+// wave's tickets are taken together after its last down item. Before, an item's loads went
+// out one item at a time through flat addresses, every pass did four tokens' sums in down,
+// and a ticket's round trip followed each item. 64 experts top-6, 2048 / 1408, f32: 97 -> 79
+// us at 6 tokens (240 MB, 37 us at the stream's rate), 173 -> 150 at 16, 305 -> 271 at 40;
+// 128 experts top-8, 4096 / 1536: 220 -> 184 at 6, 694 -> 654 at 32; bf16 at 24 576 -> 478.
+
+// A streamed 16 bytes at lane offset `off` past uniform offset `base`, which the bounds check
+// need not count: callers keep base + off inside the resource or `off` past every one.
+__device__ __forceinline__ uint4 ld16nt(__amdgpu_buffer_rsrc_t r, int off, int base) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off, base, BUF_NT);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+// A row's bytes where they are used: the compiler cannot lift their conversion out of the
+// loop over tokens (kept converted, an item's rows take 256 registers and spill).
+__device__ __forceinline__ uint4 in_place(uint4 w) {
+    asm volatile("" : "+v"(w.x), "+v"(w.y), "+v"(w.z), "+v"(w.w));
+    return w;
+}
+
+// 16 columns of one activation row through a buffer resource (zeros where off is OOB).
+template <int XDT>
+struct X16;
+template <>
+struct X16<OOM_BF16> {
+    uint32_t w[8];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int off) {
+        const uint4 a = ld16(r, off), b = ld16(r, off + 16);
+        w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w;
+        w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
+    }
+};
+template <>
+struct X16<OOM_F32> {
+    float v[16];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int off) {
 #pragma unroll
-    for (int r = 0; r < FG_R; r++) {
-        const size_t row = (size_t)min(j0 + r, I - 1) * H;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int col = c * 1024 + lane * 16;
-            const bool ok = c < CH && col < H;
-            wg[r][c] = ok ? *reinterpret_cast<const uint4*>(rec + a.gw + row + col) : make_uint4(0, 0, 0, 0);
-            wu[r][c] = ok ? *reinterpret_cast<const uint4*>(rec + a.uw + row + col) : make_uint4(0, 0, 0, 0);
+        for (int q = 0; q < 4; q++) {
+            const uint4 a = ld16(r, off + 16 * q);
+            v[4 * q] = __uint_as_float(a.x);
+            v[4 * q + 1] = __uint_as_float(a.y);
+            v[4 * q + 2] = __uint_as_float(a.z);
+            v[4 * q + 3] = __uint_as_float(a.w);
         }
     }
-    const float* gs = reinterpret_cast<const float*>(rec + a.gs) + (size_t)(j0 >> 7) * nkb;
-    const float* us = reinterpret_cast<const float*>(rec + a.us) + (size_t)(j0 >> 7) * nkb;
-    const int a_begin = pl.off[i], a_end = pl.off[i + 1];
-    for (int a0 = a_begin; a0 < a_end; a0 += TG) {
-        const int nb = min(TG, a_end - a0);
-        float acc[TG * 2 * FG_R];  // [t][gate r0, gate r1, up r0, up r1]
+};
+
+// Gate/up item `it`: FG_R gate and FG_R up rows of expert it / tiles_g, CS chunks of 1024
+// columns; an item past NG reads zeros. With one row each, the activations read per weight
+// double: 32 f32 tokens of 4096 / 1536 took 814 us against 654.
+template <int CS>
+struct GateUpW {
+    uint4 w[2 * FG_R][CS];  // gate rows, then up rows
+    float sg[CS], su[CS];
+};
+
+template <int CS>
+__device__ __forceinline__ void gate_up_load(const FusedArgs& a, const PlanLds& pl, int it, int NG, int tiles_g, int lane,
+                                             GateUpW<CS>& d) {
+    constexpr int R = FG_R;
+    const int H = (int)a.H, I = (int)a.I, nkb = (H + 127) >> 7;
+    const bool valid = it < NG;
+    const int i = __builtin_amdgcn_readfirstlane(valid ? it / tiles_g : 0);
+    const int j0 = __builtin_amdgcn_readfirstlane(valid ? (it - i * tiles_g) * R : 0);
+    const __amdgpu_buffer_rsrc_t r = rec_rsrc(pl, i, valid ? a.rec_bytes : 0);
 #pragma unroll
-        for (int q = 0; q < TG * 2 * FG_R; q++) acc[q] = 0.0f;
+    for (int c = 0; c < CS; c++) {
+        const int col = c * 1024 + lane * 16;
+        const bool ok = valid && col < H;
+        const int sc = ((j0 >> 7) * nkb + (col >> 7)) * 4;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            if (c >= CH) break;
-            const int col = c * 1024 + lane * 16;
-            const bool ok = col < H;
-            const float sg = ok ? gs[col >> 7] : 0.0f, su = ok ? us[col >> 7] : 0.0f;
-            if constexpr (XDT == OOM_BF16) {
-                // bf16 activations: e4m3 pairs -> bf16 pairs, bf16 dot2 into fp32
-#pragma unroll
-                for (int t = 0; t < TG; t++) {
-                    if (t >= nb) break;
-                    uint32_t xw[8];
-                    if (ok) {
-                        const uint4* xp = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(a.x) +
-                                                                         (size_t)pl.assign_tok[a0 + t] * H + col);
-                        const uint4 x0 = xp[0], x1 = xp[1];
-                        xw[0] = x0.x; xw[1] = x0.y; xw[2] = x0.z; xw[3] = x0.w;
-                        xw[4] = x1.x; xw[5] = x1.y; xw[6] = x1.z; xw[7] = x1.w;
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < 8; q++) xw[q] = 0u;
-                    }
-#pragma unroll
-                    for (int r = 0; r < FG_R; r++) {
-                        acc[t * 2 * FG_R + r] = fmaf(dot16_e4m3_bf16(wg[r][c], xw), sg, acc[t * 2 * FG_R + r]);
-                        acc[t * 2 * FG_R + FG_R + r] =
-                            fmaf(dot16_e4m3_bf16(wu[r][c], xw), su, acc[t * 2 * FG_R + FG_R + r]);
-                    }
-                }
-            } else {
-                float f[2 * FG_R][16];
-#pragma unroll
-                for (int r = 0; r < FG_R; r++) {
-                    e4m3x16(wg[r][c], f[r]);
-                    e4m3x16(wu[r][c], f[FG_R + r]);
-                }
-#pragma unroll
-                for (int t = 0; t < TG; t++) {
-                    if (t >= nb) break;
-                    float xv[16];
-                    if (ok) load16<XDT>(a.x, (size_t)pl.assign_tok[a0 + t] * H + col, xv);
-                    else {
-#pragma unroll
-                        for (int q = 0; q < 16; q++) xv[q] = 0.0f;
-                    }
-#pragma unroll
-                    for (int r = 0; r < 2 * FG_R; r++) {
-                        float p = 0.0f;
-#pragma unroll
-                        for (int q = 0; q < 16; q++) p = fmaf(f[r][q], xv[q], p);
-                        acc[t * 2 * FG_R + r] = fmaf(p, r < FG_R ? sg : su, acc[t * 2 * FG_R + r]);
-                    }
-                }
-            }
+        for (int q = 0; q < R; q++) {
+            const int row = min(j0 + q, I - 1) * H;
+            d.w[q][c] = ld16nt(r, ok ? col : OOB, valid ? (int)a.gw + row : 0);
+            d.w[R + q][c] = ld16nt(r, ok ? col : OOB, valid ? (int)a.uw + row : 0);
         }
-        // value v = t * 4 + r ends in lane group v (groups of 64 / (4 TG) lanes)
-        constexpr int NV = TG * 2 * FG_R, GROUP = 64 / NV;
-        float tot = wave_sum_multi<NV>(acc, lane);
-        const int v = lane / GROUP;
-        float up = __shfl(tot, (lane + FG_R * GROUP) & 63, 64);
-        if (lane % GROUP == 0 && (v % (2 * FG_R)) < FG_R) {
-            const int t = v / (2 * FG_R), r = v % (2 * FG_R), j = j0 + r;
-            if (t < nb && j < I) st_dev(&a.h[(size_t)(a0 + t) * I + j], siluf(tot) * up);
+        d.sg[c] = ldf(r, ok ? (int)a.gs + sc : OOB);
+        d.su[c] = ldf(r, ok ? (int)a.us + sc : OOB);
+    }
+}
+
+// Adds chunk c of the rows' products with NT activation pieces to acc[t][gate rows, up rows].
+template <int XDT, int CS, int NT>
+__device__ __forceinline__ void gate_up_chunk(const GateUpW<CS>& d, int c, const X16<XDT> (&x)[NT], float* acc) {
+    constexpr int R = FG_R;
+#pragma unroll
+    for (int q = 0; q < 2 * R; q++) {
+        const float sc = q < R ? d.sg[c] : d.su[c];
+        const uint4 w = in_place(d.w[q][c]);
+        if constexpr (XDT == OOM_BF16) {
+            // bf16 activations: e4m3 pairs -> bf16 pairs, bf16 dot2 into fp32
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                acc[t * 2 * R + q] = fmaf(dot16_e4m3_bf16(w, x[t].w), sc, acc[t * 2 * R + q]);
+        } else {
+            float f[16];
+            e4m3x16(w, f);
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                float p = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 16; j++) p = fmaf(f[j], x[t].v[j], p);
+                acc[t * 2 * R + q] = fmaf(p, sc, acc[t * 2 * R + q]);
+            }
         }
     }
 }
 
-// The weights of down item (i, tile): 8 rows x 2 chunks of 1024 columns per lane.
+// h of NT assignments from a0 (nb of them real) from the sums.
+template <int CS, int NT>
+__device__ __forceinline__ void gate_up_put(const FusedArgs& a, int a0, int nb, int j0, int lane,
+                                            float (&acc)[NT * 2 * FG_R]) {
+    constexpr int R = FG_R, NV = NT * 2 * R, GROUP = 64 / NV;
+    const int I = (int)a.I;
+    // value v = t * 2 R + q ends in lane group v (groups of 64 / NV lanes)
+    const float tot = wave_sum_multi<NV>(acc, lane);
+    const int v = lane / GROUP;
+    const float up = __shfl(tot, (lane + R * GROUP) & 63, 64);
+    if (lane % GROUP == 0 && (v % (2 * R)) < R) {
+        const int t = v / (2 * R), j = j0 + v % (2 * R);
+        if (t < nb && j < I) st_dev(&a.h[(size_t)(a0 + t) * I + j], siluf(tot) * up);
+    }
+}
+
+// The whole of phase 1 for one wave.
+template <int XDT, int CS>
+__device__ __forceinline__ void gate_up_phase(const FusedArgs& a, const PlanLds& pl, int n_e, int gwave, int NW, int lane) {
+    constexpr int R = FG_R, TG = 2, ES = XDT == OOM_BF16 ? 2 : 4;
+    const int H = (int)a.H;
+    const int tiles_g = (int)((a.I + R - 1) / R), NG = n_e * tiles_g;
+    const __amdgpu_buffer_rsrc_t xr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), (short)0, a.T * H * ES, BUF_FLAGS);
+    const auto xoff = [&](int as, int c) {
+        const int col = c * 1024 + lane * 16;
+        return col < H ? (__builtin_amdgcn_readfirstlane(pl.assign_tok[as]) * H + col) * ES : OOB;
+    };
+    // the wave's item from its loaded rows; the next item's loads go out behind the first
+    // token's activations
+    const auto item = [&](int it, const GateUpW<CS>& d, GateUpW<CS>& next) {
+        const int i = __builtin_amdgcn_readfirstlane(it / tiles_g), j0 = (it - i * tiles_g) * R;
+        const int a0 = __builtin_amdgcn_readfirstlane(pl.off[i]), a1 = __builtin_amdgcn_readfirstlane(pl.off[i + 1]);
+        X16<XDT> x1[CS][1];
+#pragma unroll
+        for (int c = 0; c < CS; c++) x1[c][0].load(xr, xoff(a0, c));
+        gate_up_load<CS>(a, pl, it + NW, NG, tiles_g, lane, next);
+        {
+            float acc[2 * R] = {};
+#pragma unroll
+            for (int c = 0; c < CS; c++) {
+                if (c * 1024 >= H) break;
+                gate_up_chunk<XDT, CS, 1>(d, c, x1[c], acc);
+            }
+            gate_up_put<CS, 1>(a, a0, 1, j0, lane, acc);
+        }
+        for (int as = a0 + 1; as < a1; as += TG) {
+            const int nb = min(TG, a1 - as);
+            float acc[TG * 2 * R] = {};
+#pragma unroll
+            for (int c = 0; c < CS; c++) {
+                if (c * 1024 >= H) break;
+                X16<XDT> x[TG];
+#pragma unroll
+                for (int t = 0; t < TG; t++) x[t].load(xr, t < nb ? xoff(min(as + t, a1 - 1), c) : OOB);
+                gate_up_chunk<XDT, CS, TG>(d, c, x, acc);
+                __builtin_amdgcn_sched_barrier(0);  // one chunk's activations in registers at a time
+            }
+            gate_up_put<CS, TG>(a, as, nb, j0, lane, acc);
+        }
+    };
+    GateUpW<CS> wa, wb;
+    gate_up_load<CS>(a, pl, gwave, NG, tiles_g, lane, wa);
+    for (int it = gwave; it < NG; it += 2 * NW) {
+        item(it, wa, wb);
+        if (it + NW >= NG) break;
+        item(it + NW, wb, wa);
+    }
+}
+
+// The weights and scales of down item `it` (expert it / tiles_d): 8 rows x 2 chunks of 1024
+// columns per lane; an item past ND reads zeros.
 struct DownW {
     uint4 w[FD_R][2];
+    float s[2];
 };
 
-__device__ __forceinline__ void down_load(const FusedArgs& a, const PlanLds& pl, int i, int tile, int lane, DownW& d) {
-    const int H = (int)a.H, I = (int)a.I, CH = (I + 1023) >> 10;
-    const uint8_t* rec = reinterpret_cast<const uint8_t*>(pl.recs[pl.experts[i]]);
-    const int r0 = tile * FD_R;
+__device__ __forceinline__ void down_load(const FusedArgs& a, const PlanLds& pl, int it, int ND, int tiles_d, int lane,
+                                          DownW& d) {
+    const int H = (int)a.H, I = (int)a.I, nkb = (I + 127) >> 7;
+    const bool valid = it < ND;
+    const int i = __builtin_amdgcn_readfirstlane(valid ? it / tiles_d : 0);
+    const int r0 = __builtin_amdgcn_readfirstlane(valid ? (it - i * tiles_d) * FD_R : 0);
+    const __amdgpu_buffer_rsrc_t r = rec_rsrc(pl, i, valid ? a.rec_bytes : 0);
 #pragma unroll
-    for (int r = 0; r < FD_R; r++) {
-        const size_t row = (size_t)min(r0 + r, H - 1) * I;
+    for (int c = 0; c < 2; c++) {
+        const int col = c * 1024 + lane * 16;
+        const bool ok = valid && col < I;
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const int col = c * 1024 + lane * 16;
-            d.w[r][c] = (c < CH && col < I) ? *reinterpret_cast<const uint4*>(rec + a.dw + row + col)
-                                            : make_uint4(0, 0, 0, 0);
-        }
+        for (int q = 0; q < FD_R; q++)
+            d.w[q][c] = ld16nt(r, ok ? col : OOB, valid ? (int)a.dw + min(r0 + q, H - 1) * I : 0);
+        d.s[c] = ldf(r, ok ? (int)a.ds + ((r0 >> 7) * nkb + (col >> 7)) * 4 : OOB);
     }
 }
 
@@ -233,62 +311,49 @@ __device__ __forceinline__ void down_load(const FusedArgs& a, const PlanLds& pl,
 // columns, through device-coherent 128-bit buffer loads.
 template <int TG>
 __device__ __forceinline__ void down_h_load(const FusedArgs& a, int a0, int nb, int lane, float (&hv)[TG][2][16]) {
-    const int I = (int)a.I, CH = (I + 1023) >> 10;
-    const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(a.h, (short)0, a.h_bytes, 0x00020000);
+    const int I = (int)a.I;
+    const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(a.h, (short)0, a.h_bytes, BUF_FLAGS);
 #pragma unroll
     for (int t = 0; t < TG; t++)
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int col = c * 1024 + lane * 16;
-            if (t < nb && c < CH && col < I) {
-                const int off = (int)(((size_t)(a0 + t) * I + col) * sizeof(float));
+            const int off = t < nb && col < I ? ((a0 + t) * I + col) * 4 : OOB;
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const auto v = __builtin_amdgcn_raw_buffer_load_b128(hr, off + 16 * q, 0, BUF_SC1);
-                    hv[t][c][4 * q] = __uint_as_float(v[0]);
-                    hv[t][c][4 * q + 1] = __uint_as_float(v[1]);
-                    hv[t][c][4 * q + 2] = __uint_as_float(v[2]);
-                    hv[t][c][4 * q + 3] = __uint_as_float(v[3]);
-                }
-            } else {
-#pragma unroll
-                for (int q = 0; q < 16; q++) hv[t][c][q] = 0.0f;
+            for (int q = 0; q < 4; q++) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(hr, off + 16 * q, 0, BUF_SC1);
+                hv[t][c][4 * q] = __uint_as_float(v[0]);
+                hv[t][c][4 * q + 1] = __uint_as_float(v[1]);
+                hv[t][c][4 * q + 2] = __uint_as_float(v[2]);
+                hv[t][c][4 * q + 3] = __uint_as_float(v[3]);
             }
         }
 }
 
 // y[a0 + t, r0 .. r0 + FD_R) = h . Wd rows for the token group, from loaded weights and h.
 template <int TG>
-__device__ __forceinline__ void down_rows(const FusedArgs& a, const PlanLds& pl, int i, int tile, int lane,
-                                          const DownW& d, const float (&hv)[TG][2][16], int a0, int nb) {
-    const int H = (int)a.H, I = (int)a.I;
-    const int CH = (I + 1023) >> 10, nkb = (I + 127) >> 7;
-    const uint8_t* rec = reinterpret_cast<const uint8_t*>(pl.recs[pl.experts[i]]);
-    const int r0 = tile * FD_R;
-    const float* ds = reinterpret_cast<const float*>(rec + a.ds) + (size_t)(r0 >> 7) * nkb;
-    float acc[TG * FD_R];
-#pragma unroll
-    for (int q = 0; q < TG * FD_R; q++) acc[q] = 0.0f;
+__device__ __forceinline__ void down_rows(const FusedArgs& a, int r0, int lane, const DownW& d,
+                                          const float (&hv)[TG][2][16], int a0, int nb) {
+    const int H = (int)a.H;
+    float acc[TG * FD_R] = {};
 #pragma unroll
     for (int c = 0; c < 2; c++) {
-        if (c >= CH) break;
-        const int col = c * 1024 + lane * 16;
-        const float sd = col < I ? ds[col >> 7] : 0.0f;
+        if (c * 1024 >= (int)a.I) break;
 #pragma unroll
         for (int r = 0; r < FD_R; r++) {
             float f[16];
-            e4m3x16(d.w[r][c], f);
+            e4m3x16(in_place(d.w[r][c]), f);
 #pragma unroll
             for (int t = 0; t < TG; t++) {
                 float p = 0.0f;
 #pragma unroll
                 for (int q = 0; q < 16; q++) p = fmaf(f[q], hv[t][c][q], p);
-                acc[t * FD_R + r] = fmaf(p, sd, acc[t * FD_R + r]);
+                acc[t * FD_R + r] = fmaf(p, d.s[c], acc[t * FD_R + r]);
             }
         }
     }
     constexpr int NV = TG * FD_R, GROUP = 64 / NV;
-    float tot = wave_sum_multi<NV>(acc, lane);
+    const float tot = wave_sum_multi<NV>(acc, lane);
     const int v = lane / GROUP;
     if (lane % GROUP == 0) {
         const int t = v / FD_R, r = r0 + v % FD_R;
@@ -297,7 +362,7 @@ __device__ __forceinline__ void down_rows(const FusedArgs& a, const PlanLds& pl,
 }
 
 // Combine of output row tile `tile` for every token, in slot order, by the wave that
-// took the tile's last ticket; it then resets the ticket.
+// took the tile's last ticket; it then resets the ticket. Eight slots' loads go out together.
 template <int ODT>
 __device__ __forceinline__ void combine_tile(const FusedArgs& a, const PlanLds& pl, int tile, int lane) {
     const int H = (int)a.H, r0 = tile * FD_R;
@@ -305,44 +370,74 @@ __device__ __forceinline__ void combine_tile(const FusedArgs& a, const PlanLds& 
         const int t = idx / FD_R, r = r0 + idx % FD_R;
         if (r >= H) continue;
         float acc = 0.0f;
-        for (int s = 0; s < a.k; s++)
-            acc = fmaf(pl.w[t * a.k + s], ld_dev(&a.y[(size_t)pl.slot_assign[t * a.k + s] * H + r]), acc);
+        for (int s0 = 0; s0 < a.k; s0 += 8) {
+            float v[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                v[q] = ld_dev(&a.y[(size_t)pl.slot_assign[t * a.k + min(s0 + q, a.k - 1)] * H + r]);
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                if (s0 + q < a.k) acc = fmaf(pl.w[t * a.k + s0 + q], v[q], acc);
+        }
         store_out<ODT>(a.out, (size_t)t * H + r, acc);
     }
     if (lane == 0) __hip_atomic_store(&a.tickets[tile * TICKET_STRIDE], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Takes a ticket of row tile `tile` (after this wave's y stores completed); true if it
-// was the tile's last (every expert's rows of the tile are in y).
-__device__ __forceinline__ uint32_t take_ticket(const FusedArgs& a, int tile, int lane) {
-    uint32_t old = 0;
-    if (lane == 0)
-        old = __hip_atomic_fetch_add(&a.tickets[tile * TICKET_STRIDE], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return old;
-}
-
-// Down item (i, tile) over all of the expert's tokens, weights already loaded.
-template <int TG>
-__device__ __forceinline__ void down_item(const FusedArgs& a, const PlanLds& pl, int i, int tile, int lane,
-                                          const DownW& d) {
-    const int a_begin = pl.off[i], a_end = pl.off[i + 1];
-    for (int a0 = a_begin; a0 < a_end; a0 += TG) {
-        const int nb = min(TG, a_end - a0);
-        float hv[TG][2][16];
-        down_h_load<TG>(a, a0, nb, lane, hv);
-        down_rows<TG>(a, pl, i, tile, lane, d, hv, a0, nb);
+// Phase 2 for one wave, its first item's weights already loading in wa: the y rows of its
+// items, then the tickets of their row tiles (a lane each, 64 items at a time) once the
+// wave's y stores completed; the taker of a tile's last ticket combines it.
+template <int ODT>
+__device__ __forceinline__ void down_phase(const FusedArgs& a, const PlanLds& pl, int n_e, int ND, int tiles_d, int gwave,
+                                           int NW, int lane, DownW& wa) {
+    const auto item = [&](int it, const DownW& d, DownW& next) {
+        const int i = __builtin_amdgcn_readfirstlane(it / tiles_d), r0 = (it - i * tiles_d) * FD_R;
+        const int a0 = __builtin_amdgcn_readfirstlane(pl.off[i]), a1 = __builtin_amdgcn_readfirstlane(pl.off[i + 1]);
+        {
+            float hv[1][2][16];
+            down_h_load<1>(a, a0, 1, lane, hv);
+            down_load(a, pl, it + NW, ND, tiles_d, lane, next);
+            down_rows<1>(a, r0, lane, d, hv, a0, 1);
+        }
+        for (int as = a0 + 1; as < a1; as += 2) {
+            const int nb = min(2, a1 - as);
+            float hv[2][2][16];
+            down_h_load<2>(a, as, nb, lane, hv);
+            down_rows<2>(a, r0, lane, d, hv, as, nb);
+        }
+    };
+    const auto flush = [&](int first, int n) {  // the tickets of items first, first + NW, ... (n <= 64)
+        wait_mem();
+        uint32_t old = 0;
+        const int tile = (first + lane * NW) % tiles_d;
+        if (lane < n)
+            old = __hip_atomic_fetch_add(&a.tickets[tile * TICKET_STRIDE], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint64_t last = __ballot(lane < n && old == (uint32_t)n_e - 1);
+        while (last) {
+            const int l = __builtin_ctzll(last);
+            last &= last - 1;
+            combine_tile<ODT>(a, pl, __builtin_amdgcn_readlane(tile, l), lane);
+        }
+    };
+    DownW wb;
+    int first = gwave, n = 0;
+    for (int it = gwave; it < ND; it += 2 * NW) {
+        item(it, wa, wb);
+        n++;
+        if (it + NW < ND) {
+            item(it + NW, wb, wa);
+            n++;
+        }
+        if (n == 64) {
+            flush(first, n);
+            first = it + 2 * NW;
+            n = 0;
+        }
     }
+    if (n) flush(first, n);
 }
 
 // ---- one token (T == 1) ------------------------------------------------------------------
-
-// A record's parts through one buffer resource; an empty resource (bytes 0) reads zeros.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rec_rsrc(const PlanLds& pl, int i, int bytes) {
-    const uint64_t r = pl.recs[pl.experts[i]];
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)r), hi = __builtin_amdgcn_readfirstlane((uint32_t)(r >> 32));
-    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), (short)0, bytes,
-                                             BUF_FLAGS);
-}
 
 // Gate/up item `it` (plan slot item_slot(it), row it % I): one gate row and one up row,
 // 1024 columns per chunk, and their 128 x 128-block scales; an item past NG reads zeros.
@@ -606,7 +701,7 @@ __device__ __forceinline__ void plan_wave(PlanLds& pl, int A, int k, int lane) {
 }
 
 template <int TG, int DCH, int EQ, int XDT, int ODT, bool SH = false>
-__global__ void __launch_bounds__(TG == 1 ? 64 * FW1 : 64 * FW) moe_decode_fused_kernel(FusedArgs a) {
+__global__ void __launch_bounds__(TG == 1 ? 64 * FW1 : 64 * FW, 2) moe_decode_fused_kernel(FusedArgs a) {
     static_assert(!SH || TG == 1, "the shared expert rides the one-token kernel");
     constexpr int WB = TG == 1 ? FW1 : FW;  // waves per block
     __shared__ PlanLds pl;
@@ -824,22 +919,15 @@ __global__ void __launch_bounds__(TG == 1 ? 64 * FW1 : 64 * FW) moe_decode_fused
         }
         OOM_STAMP(a.stamps, WB, 6);  // combined and stored
     } else {
-        // ---- phase 1: gate/up + SwiGLU -> h, FG_R rows per item, tokens in groups of TG ----
-        const int tiles_g = (int)((a.I + FG_R - 1) / FG_R), NG = n_e * tiles_g;
-        for (int it = gwave; it < NG; it += NW) gate_up_item<TG, XDT>(a, pl, it / tiles_g, it % tiles_g, lane);
+        // ---- phase 1: gate/up + SwiGLU -> h ----
+        gate_up_phase<XDT, DCH>(a, pl, n_e, gwave, NW, lane);
         wait_mem();  // this wave's h stores are complete before its block arrives
         // ---- the first down item's weights stream while the grid meets ----
         DownW d;
-        if (gwave < ND) down_load(a, pl, gwave / tiles_d, gwave % tiles_d, lane, d);
+        down_load(a, pl, gwave, ND, tiles_d, lane, d);
         grid_barrier(a, bbase);
         // ---- phase 2: down projection -> y, then the ticketed slot-order combine ----
-        for (int it = gwave; it < ND; it += NW) {
-            if (it != gwave) down_load(a, pl, it / tiles_d, it % tiles_d, lane, d);
-            down_item<TG>(a, pl, it / tiles_d, it % tiles_d, lane, d);
-            wait_mem();
-            if ((uint32_t)__builtin_amdgcn_readlane((int)take_ticket(a, it % tiles_d, lane), 0) == (uint32_t)n_e - 1)
-                combine_tile<ODT>(a, pl, it % tiles_d, lane);
-        }
+        down_phase<ODT>(a, pl, n_e, ND, tiles_d, gwave, NW, lane, d);
     }
     grid_barrier_exit(a.bar);
 }
@@ -953,7 +1041,7 @@ int launch_fused(const float* logits, const void* x, int xdt, const uint64_t* al
     if (xdt == OOM_F32 && odt == OOM_BF16) return launch_fused_t<TG, DCH, EQ, OOM_F32, OOM_BF16>(a, lds, st);   \
     return launch_fused_t<TG, DCH, EQ, OOM_F32, OOM_F32>(a, lds, st);
     // one token routed to at most FW1 experts: TG 1 with 512-column down chunks for the
-    // inter width; otherwise groups of 4 tokens per pass over an item's weights
+    // inter width; otherwise TG 4 with 1024-column chunks for the hidden width
     if (T == 1 && k <= FW1) {
         if (E <= 128) {
             if (g.inter <= 1024) {
@@ -972,8 +1060,10 @@ int launch_fused(const float* logits, const void* x, int xdt, const uint64_t* al
                 FUSED_CASE(1, 4, 4)
             }
         }
+    } else if (g.hidden <= 2048) {
+        FUSED_CASE(4, 2, 4)
     } else {
-        FUSED_CASE(4, 0, 4)
+        FUSED_CASE(4, 4, 4)
     }
 #undef FUSED_CASE
 }

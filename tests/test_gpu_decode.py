@@ -305,6 +305,13 @@ def test_fused_decode_full_size(hip, T, E, k, zipf, H, I):
     (1, 16, 9, 256, 128, False),     # one token, more experts than the one-token kernel's waves
     (1, 64, 12, 512, 256, True),
     (1, 256, 32, 1040, 272, False),  # the most picks; widths ending inside a chunk
+    (2, 16, 2, 16, 16, True),        # the smallest widths: most waves without an item
+    (6, 64, 6, 2048, 1408, True),    # two chunks a row, mostly one token an expert
+    (5, 8, 8, 2064, 1040, True),     # four chunks, one row an item; odd groups; tiles past a chunk's end
+    (33, 8, 2, 1008, 272, False),    # bf16 past the batch kernel
+    (64, 4, 4, 4096, 144, True),     # the widest rows, every token on every expert, more down tiles than waves
+    (20, 96, 8, 3072, 2048, False),  # bf16, four chunks, the widest inter
+    (40, 32, 12, 512, 1024, True),   # A = 480; combine past eight slots
 ])
 def test_fused_decode_general(hip, T, E, k, H, I, xf32):
     """The one-launch kernel for what the one-token and the MFMA batch kernels leave: one
