@@ -545,7 +545,9 @@ __global__ void __launch_bounds__(64 * N4S_WAVES) moe_gate_up_nvfp4_step_kernel(
     __shared__ Plan4Lds pl;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int H = g.H, I = g.I, CH = (H + 1023) >> 10;
-    const int ipe = (I + 2 * N4_GP - 1) / (2 * N4_GP), NG = *n_e_dev * ipe, NW = gridDim.x * N4S_WAVES;
+    const int n_e = *n_e_dev;
+    if (n_e <= 0) return;  // the plan found an id that is no expert
+    const int ipe = (I + 2 * N4_GP - 1) / (2 * N4_GP), NG = n_e * ipe, NW = gridDim.x * N4S_WAVES;
     // items it0, it0 + NW, ...: neighbouring items on different CUs
     int it = wave * gridDim.x + blockIdx.x;
     const auto rsrc_of = [&](int item, uint64_t rec) { return uniform_rsrc(rec, item < NG ? g.bytes : 0); };
@@ -555,7 +557,6 @@ __global__ void __launch_bounds__(64 * N4S_WAVES) moe_gate_up_nvfp4_step_kernel(
         gu4_load<CS>(g, rsrc_of(it, recs[e]), (it - e * ipe) * 2 * N4_GP, lane, 0, ta);
     }
     // the plan and every token's x into LDS (stage4's lane order)
-    const int n_e = *n_e_dev;
     if ((int)threadIdx.x < n_e) {
         const int e = threadIdx.x;
         const uint64_t rec = recs[e];
