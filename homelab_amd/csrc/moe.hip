@@ -325,6 +325,8 @@ int launch_combine(const float* y, const int32_t* slot, const float* w, void* ou
 static bool lds_fits(int64_t width) { return (size_t)MOE_TB * cdiv(width, 1024) * 1024 * sizeof(float) <= 65536; }
 
 // The one-launch path (moe_fused.hip) and its workspace.
+int launch_route_plan(const float* logits, int T, int E, int k, const uint64_t* all_recs, int32_t* ids, float* weights,
+                      int32_t* plan, uint64_t* recs, hipStream_t st);
 bool fused_supported(int T, int E, int k, const OomFp8Record& g);
 size_t fused_workspace_size(int T, int E, int k, const OomFp8Record& g);
 int launch_fused(const float* logits, const void* x, int xdt, const uint64_t* all_recs, int T, int E, int k,
@@ -424,8 +426,7 @@ extern "C" int oom_moe_decode_fp8(const float* logits, const void* x, int x_dtyp
     hipStream_t st = as_stream(stream);
     const int A = T * k;
     PlanView pv{plan, E, A};
-    if (int rc = oom_router_topk(logits, ids, weights, T, E, k, stream)) return rc;
-    if (int rc = oom_moe_plan(ids, T, E, k, all_recs, plan, recs, stream)) return rc;
+    if (int rc = launch_route_plan(logits, T, E, k, all_recs, ids, weights, plan, recs, st)) return rc;
     const int grid_e = std::min(E, A);
     if (int rc = launch_gate_up(recs, pv.off(), pv.assign_tok(), grid_e, x, x_dtype, h, *geo, pv.n_e(), st)) return rc;
     if (int rc = launch_down(recs, pv.off(), grid_e, h, y, *geo, pv.n_e(), st)) return rc;

@@ -27,12 +27,10 @@
 #include "router.hpp"
 #include "stream.hpp"
 
-extern "C" int oom_router_topk(const float* logits, int32_t* ids, float* weights, int T, int E, int k, void* stream);
-extern "C" int oom_moe_plan(const int32_t* ids, int T, int E, int k, const uint64_t* all_recs, int32_t* plan,
-                            uint64_t* recs, void* stream);
-
 namespace oom {
 
+int launch_route_plan(const float* logits, int T, int E, int k, const uint64_t* all_recs, int32_t* ids, float* weights,
+                      int32_t* plan, uint64_t* recs, hipStream_t st);
 int launch_combine(const float* y, const int32_t* slot, const float* w, void* out, int odt, int T, int H, int k,
                    hipStream_t st);
 
@@ -1103,8 +1101,7 @@ extern "C" int oom_moe_decode_nvfp4(const float* logits, const void* x, int x_dt
     }
     const int A = T * k;
     const PlanView pv{plan, E, A};
-    if (int rc = oom_router_topk(logits, ids, weights, T, E, k, stream)) return rc;
-    if (int rc = oom_moe_plan(ids, T, E, k, all_recs, plan, recs, stream)) return rc;
+    if (int rc = launch_route_plan(logits, T, E, k, all_recs, ids, weights, plan, recs, st)) return rc;
     const int grid_e = std::min(E, A);
     if (gate_up_step_ok(T, A, grid_e, *geo)) {
         if (int rc = launch_gate_up_step(recs, pv, x, x_dtype, T, h, *geo, st)) return rc;

@@ -228,6 +228,7 @@ __global__ void __launch_bounds__(1024) moe_plan_kernel(const int32_t* __restric
 }  // namespace oom
 extern "C" int oom_moe_plan(const int32_t* ids, int T, int E, int k, const uint64_t* all_recs, int32_t* plan,
                             uint64_t* recs, void* stream);
+extern "C" int oom_router_topk(const float* logits, int32_t* ids, float* weights, int T, int E, int k, void* stream);
 namespace oom {
 
 // ---- the plan over many blocks (large steps, E <= PLAN_FAST_E) -------------------------
@@ -422,6 +423,103 @@ int launch_plan_multi(const int32_t* ids, int T, int E, int k, const uint64_t* a
     hipLaunchKernelGGL(plan_place_kernel, dim3(NB), dim3(PM_THREADS), (PM_WAVES + 1) * E * sizeof(int), st, ids, A, E,
                        k, C, NB, counts, all_recs, plan, recs);
     return launched("oom_moe_plan");
+}
+
+// ---- routing and plan of a few tokens in one launch -------------------------------------
+//
+// Both are chains of short latencies (6.4 us and 8 us as two launches at 8 tokens, 512
+// experts, top-10), so one block does both: a wave routes a token (route_token_regs), and
+// with the ids in LDS every slot's place comes from comparisons with all slots, P = 1024 /
+// (slots rounded up to a power of two) threads a slot: no counts, scans or rounds. NVFP4
+// decode step: 40.0 -> 35.1 us at 2 tokens of that, 87.9 -> 85 at 8, 20.0 -> 15.6 at 2 tokens
+// of 64 experts top-4, 1024 / 256.
+// The line: past two tokens a SIMD the one CU routes slower than a block a token does (16
+// tokens of 256 experts top-6, 1024 / 256: 38.2 against 37.4 us; of 512 top-10: 167 and 163).
+constexpr int RP_T = 8;      // a wave a token
+constexpr int RP_A = 96;     // slots
+constexpr int RP_LDS = 128;  // slots rounded up to 4 P
+template <int EQ>
+__global__ void __launch_bounds__(1024) route_plan_kernel(const float* __restrict__ logits, int T, int E, int k,
+                                                          const uint64_t* __restrict__ all_recs,
+                                                          int32_t* __restrict__ ids, float* __restrict__ weights,
+                                                          int32_t* plan_base, uint64_t* __restrict__ recs) {
+    __shared__ int4 id_s4[RP_LDS / 4], first_s4[RP_LDS / 4];
+    int* id_s = reinterpret_cast<int*>(id_s4);
+    int* first_s = reinterpret_cast<int*>(first_s4);
+    __shared__ int bad;
+    const int A = T * k, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    PlanView plan{plan_base, E, A};
+    constexpr int NONE = 0x7fffffff;  // past every id
+    if (tid == 0) bad = 0;
+    if (tid < RP_LDS) id_s[tid] = first_s[tid] = NONE;
+    __syncthreads();
+    if (wave < T) {
+        int id = 0;
+        float w = 0.0f;
+        route_token_regs<EQ>(logits + (size_t)wave * E, E, k, lane, id, w);
+        if (lane < k) {
+            ids[wave * k + lane] = id;
+            weights[wave * k + lane] = w;
+            id_s[wave * k + lane] = id;
+            if (id < 0 || id >= E) bad = 1;
+        }
+    }
+    __syncthreads();
+    if (bad) {
+        if (tid == 0) *plan.n_e() = -1;
+        return;
+    }
+    const int lg = A <= 64 ? 4 : 3, P = 1 << lg;
+    const int s = tid >> lg, part = tid & (P - 1);
+    const auto group_sum = [&](int v) {
+        for (int o = 1; o < P; o <<= 1) v += __shfl_xor(v, o, 64);
+        return v;
+    };
+    const int e = s < A ? id_s[s] : NONE;
+    int below = 0, before = 0;  // slots of lower ids; earlier slots of this id
+    for (int j = 4 * part; j < A; j += 4 * P) {
+        const int4 v = id_s4[j >> 2];
+        below += (v.x < e) + (v.y < e) + (v.z < e) + (v.w < e);
+        before += (v.x == e && j < s) + (v.y == e && j + 1 < s) + (v.z == e && j + 2 < s) + (v.w == e && j + 3 < s);
+    }
+    below = group_sum(below);
+    before = group_sum(before);
+    const bool mine = s < A && part == 0, first = mine && before == 0;
+    const uint64_t rec = first ? all_recs[e] : 0;
+    if (mine) first_s[s] = first ? e : NONE;
+    __syncthreads();
+    int x = 0, n_e = 0;  // experts below this id; experts
+    for (int j = 4 * part; j < A; j += 4 * P) {
+        const int4 v = first_s4[j >> 2];
+        x += (v.x < e) + (v.y < e) + (v.z < e) + (v.w < e);
+        n_e += (v.x != NONE) + (v.y != NONE) + (v.z != NONE) + (v.w != NONE);
+    }
+    x = group_sum(x);
+    n_e = group_sum(n_e);
+    if (mine) {
+        plan.slot_assign()[s] = below + before;
+        plan.assign_tok()[below + before] = s / k;
+    }
+    if (first) {
+        plan.experts()[x] = e;
+        plan.off()[x] = below;
+        recs[x] = rec;
+    }
+    for (int i = n_e + tid; i < E; i += 1024) plan.experts()[i] = -1;
+    for (int i = n_e + tid; i <= E; i += 1024) plan.off()[i] = A;
+    if (tid == 0) *plan.n_e() = n_e;
+}
+
+// oom_router_topk and oom_moe_plan of a step whose arguments those accept.
+int launch_route_plan(const float* logits, int T, int E, int k, const uint64_t* all_recs, int32_t* ids, float* weights,
+                      int32_t* plan, uint64_t* recs, hipStream_t st) {
+    if (T > RP_T || T * k > RP_A || E > 512) {
+        if (int rc = oom_router_topk(logits, ids, weights, T, E, k, st)) return rc;
+        return oom_moe_plan(ids, T, E, k, all_recs, plan, recs, st);
+    }
+    hipLaunchKernelGGL(E <= 256 ? route_plan_kernel<4> : route_plan_kernel<8>, dim3(1), dim3(1024), 0, st, logits, T, E, k,
+                       all_recs, ids, weights, plan, recs);
+    return launched("oom_moe_route_plan");
 }
 
 }  // namespace oom

@@ -255,6 +255,10 @@ def _one_launch_check(hip, E, k, H, I, xf32, seed, logits):
     (32, 128, 16, 1008, 304, 2.0, False),  # A = 512, the plan's most, experts with many tokens
     (33, 128, 16, 1008, 304, 2.0, False),  # A = 528: the staged launch
     (7, 256, 4, 2048, 1552, 0.0, True),    # all logits equal: every token on the same four experts
+    (8, 300, 12, 256, 128, 2.0, False),    # routed and planned in one launch: its most tokens and slots
+    (9, 257, 3, 256, 128, 2.0, False),     # ... one token past it
+    (2, 33, 32, 256, 128, 2.0, True),      # ... A = 64; most experts chosen by both
+    (5, 64, 13, 256, 128, 2.0, True),      # ... A = 65: fewer threads a slot
 ])
 def test_decode_nvfp4_step_matches_stages(hip, T, E, k, H, I, levels, xf32):
     """Several tokens: the step's gate/up stages all of x per block and free-runs its waves
