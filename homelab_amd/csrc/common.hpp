@@ -7,6 +7,7 @@
 #include <string>
 
 #include "../../include/oom_hip.h"
+#include "dispatch.hpp"
 
 namespace oom {
 
@@ -30,7 +31,6 @@ uint32_t wait_limit();
     } while (0)
 
 inline bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
-inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 // ---- number formats ---------------------------------------------------------------

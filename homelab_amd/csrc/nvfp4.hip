@@ -524,8 +524,6 @@ __device__ __forceinline__ void dn4_compute(const Dn4W& w, const float4* xs4, co
 // arithmetic is gu4_math's, so every output has the staged kernel's bits. Down stays staged:
 // the same form of it re-reads an expert's h per wave and took 39 us against 30.
 constexpr int N4S_WAVES = 8;
-constexpr int N4S_AMAX = 512;               // assignments of a step (and so routed experts)
-constexpr size_t N4S_XMAX = 144 * 1024;     // of LDS for the tokens' x, beside the plan's 12 KiB
 
 // The step's plan as the waves read it.
 struct Plan4Lds {
@@ -964,23 +962,10 @@ static int launch_gate_up4(const uint64_t* recs, const int32_t* off, const int32
     return launched("oom_moe_gate_up_nvfp4");
 }
 
-// A step whose tokens' x fits LDS beside the plan, with rows enough (the most that its
-// assignments can reach) to pay for staging all of x in every block. The whole step, staged
-// against this: 64 experts of 1040 / 272 (18 M) 35.6 and 38.3 us, 8 of 1024 / 256 (2 M) 20.0
-// and 20.9; 20 of 2560 / 640 (33 M) 40.4 and 40.0, 80 (131 M) 97 and 86, 144 of 2560 / 1536
-// (566 M) 113 and 95.
-constexpr int64_t N4S_MIN_ROWS = 24ll << 20;  // experts x hidden x inter
-static size_t gate_up_step_lds(int T, const OomNvfp4Record& g) {
-    return (size_t)((T + 1) / 2 * 2) * cdiv(g.hidden, 1024) * 4096;  // staged two rows at a time
-}
-static bool gate_up_step_ok(int T, int A, int grid_e, const OomNvfp4Record& g) {
-    return A <= N4S_AMAX && gate_up_step_lds(T, g) <= N4S_XMAX && grid_e * g.hidden * g.inter >= N4S_MIN_ROWS;
-}
-
 template <int XDT, int CS>
 static int launch_gate_up_step_t(const uint64_t* recs, const PlanView& pv, const void* x, int T, float* h,
                                  const OomNvfp4Record& geo, hipStream_t st) {
-    const size_t lds = gate_up_step_lds(T, geo);
+    const size_t lds = (size_t)gate_up_step_lds(T, geo.hidden);
     static thread_local int raised_dev = -1;  // the device whose limit on dynamic LDS was raised
     int dev = 0;
     (void)hipGetDevice(&dev);
@@ -1103,7 +1088,7 @@ extern "C" int oom_moe_decode_nvfp4(const float* logits, const void* x, int x_dt
     const PlanView pv{plan, E, A};
     if (int rc = launch_route_plan(logits, T, E, k, all_recs, ids, weights, plan, recs, st)) return rc;
     const int grid_e = std::min(E, A);
-    if (gate_up_step_ok(T, A, grid_e, *geo)) {
+    if (gate_up_step_ok(T, E, k, geo->hidden, geo->inter)) {
         if (int rc = launch_gate_up_step(recs, pv, x, x_dtype, T, h, *geo, st)) return rc;
     } else if (int rc = launch_gate_up4(recs, pv.off(), pv.assign_tok(), grid_e, x, x_dtype, h, *geo, pv.n_e(), st)) {
         return rc;

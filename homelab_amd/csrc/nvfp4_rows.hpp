@@ -32,11 +32,6 @@ typedef __bf16 n4bf16x2 __attribute__((ext_vector_type(2)));
 typedef float n4f32x2 __attribute__((ext_vector_type(2)));
 typedef float n4f4 __attribute__((ext_vector_type(4)));
 
-constexpr int NR_WAVES = 8;
-constexpr int NR_BATCH = 8;    // subtiles a wave between two meetings of the slices
-constexpr int NR_MAXK = 2560;  // 8 slices of 10 steps: 120 registers of activation terms
-constexpr int NR_M = 16;       // activation rows
-
 // Two f32 values as packed bf16 (round to nearest even).
 __device__ __forceinline__ uint32_t n4_cvt(float lo, float hi) {
     const n4f32x2 v = {lo, hi};
@@ -51,17 +46,6 @@ __device__ __forceinline__ n4bf16x8 n4_decode8(uint32_t cw, float sc) {
     const auto p3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw, 1.0f, 3);
     return __builtin_bit_cast(n4bf16x8, make_uint4(n4_cvt(p0[0] * sc, p0[1] * sc), n4_cvt(p1[0] * sc, p1[1] * sc),
                                                    n4_cvt(p2[0] * sc, p2[1] * sc), n4_cvt(p3[0] * sc, p3[1] * sc)));
-}
-
-// How K is split: KS = 1 << ks_log slices of 32 ST columns, the other waves on other weight rows.
-struct RowsSplit {
-    int ks_log, st;
-};
-inline RowsSplit rows_split(int64_t K) {
-    RowsSplit s{0, 10};
-    while (s.ks_log < 3 && K > (int64_t)320 << s.ks_log) s.ks_log++;
-    s.st = std::max(6, 2 * (int)cdiv(K, (int64_t)64 << s.ks_log));
-    return s;
 }
 
 // The lane's activations as A operands: columns kq .. of the K floats at `row`. RAG: the run

@@ -28,9 +28,6 @@
 
 namespace oom {
 
-constexpr int T4_BN = 128;       // weight rows a block
-constexpr int T4_BM = 64;        // assignments a block
-constexpr int T4_BK = 32;        // K step
 constexpr int T4_THREADS = 256;  // 4 waves, 32 weight rows each
 constexpr int T4_NX = T4_BM * T4_BK / 4 / T4_THREADS;  // activation float4s a thread loads a step
 constexpr int T4_LS = 40;        // LDS row stride in bf16: 32 + 8
@@ -227,12 +224,9 @@ __global__ void __launch_bounds__(T4_THREADS, 2) moe_tiled_nvfp4_kernel(TiledArg
 // operand read fall in distinct bank groups), and each wave decodes its own weights in
 // registers: e2m1 -> f32 (v_cvt_scalef32_pk_f32_fp4 at scale 1), times the e4m3 group
 // scale, -> bf16 (exact, as above). K must be a multiple of 128.
-constexpr int TW_BN = 640;       // weight rows a block
 constexpr int TW_NS = 5;         // N subtiles a wave
-constexpr int TW_BK = 128;       // K block
 constexpr int TW_THREADS = 512;  // 8 waves
 constexpr int TW_LS = 136;       // LDS row stride in bf16 (272 bytes)
-constexpr int TW_BM = 48;        // assignments a block (three M subtiles)
 constexpr int TW_MS = TW_BM / 16;
 
 template <int TERMS>
@@ -491,30 +485,6 @@ __global__ void __launch_bounds__(64 * NR_WAVES) moe_tiled_nvfp4_rows_kernel(Til
     }
 }
 
-static int rows_batches(int64_t N, const RowsSplit& sp) {
-    return (int)cdiv(N, 16 * NR_BATCH * (NR_WAVES >> sp.ks_log));
-}
-
-// Where the rows kernel is the better one: K in whole scale groups a lane and at most 8 slices
-// of 10 steps, and either slices and batches that K and N fill (five sixths at least) or tiles
-// of so few rows that the stream counts and not the steps. Us a call of gate, up, SwiGLU, down
-// and combine at 2560 / 640, exact, rows kernel and tiles: 512 experts top-10, 60 tokens 287
-// and 601, 250 398 and 698, 500 451 and 722, 900 664 and 761, 1050 766 and 782, 1400 924 and
-// 1224, 2048 1218 and 1472; 64 experts, 300 tokens 228 and 296, 1200 612 and 626. At 1600 / 448
-// (slices 78 % and 88 % full) 128 experts top-4, 600 tokens 151 and 185, but 64 experts top-10,
-// 1200 tokens (190 rows an expert) 398 and 327. The tiles also keep the steps of many experts
-// whose 41 to 48 rows at most are one 48-row tile where the rows kernel decodes twice or more
-// (512 experts, 1200 tokens: 815 and 786; with 128 experts 264 and 299).
-static bool rows_kernel_serves(int64_t N, int64_t K, int64_t w_off, int64_t s_off, int64_t n_experts, int64_t max_n,
-                               bool exact) {
-    if (K % 64 != 0 || K > NR_MAXK || w_off % 4 != 0 || s_off % 4 != 0) return false;
-    const RowsSplit sp = rows_split(K);
-    if (n_experts * cdiv(max_n, NR_M) * rows_batches(N, sp) > INT32_MAX) return false;
-    if (exact && K % TW_BK == 0 && n_experts >= 384 && max_n > 40 && max_n <= TW_BM) return false;
-    const int64_t rows = (int64_t)16 * NR_BATCH * (NR_WAVES >> sp.ks_log) * rows_batches(N, sp);
-    return 6 * K * N >= 5 * ((int64_t)32 * sp.st << sp.ks_log) * rows || max_n <= 48;
-}
-
 template <int TERMS>
 static void launch_tiled_rows(const TiledArgs& a, int n_experts, int max_per_expert, hipStream_t st) {
     const RowsSplit sp = rows_split(a.K);
@@ -562,15 +532,13 @@ extern "C" int oom_moe_tiled_nvfp4(const uint64_t* recs, const int32_t* off, con
     OOM_REQUIRE(recs && off && x && y, "oom_moe_tiled_nvfp4: null buffer");
     OOM_REQUIRE(aligned(x, 16), "oom_moe_tiled_nvfp4: x must be 16-byte aligned");
     TiledArgs a{recs, off, rows, x, y, n, k, w_off, s_off, s2_idx};
-    if (rows_kernel_serves(n, k, w_off, s_off, n_experts, max_per_expert,
-                           precision == OOM_EXPERT_EXACT)) {
+    const TiledRoute route = tiled_route(n, k, w_off, s_off, n_experts, max_per_expert, precision == OOM_EXPERT_EXACT);
+    if (route == TiledRoute::rows) {
         if (precision == OOM_EXPERT_EXACT) launch_tiled_rows<3>(a, n_experts, max_per_expert, as_stream(stream));
         else launch_tiled_rows<1>(a, n_experts, max_per_expert, as_stream(stream));
         return launched("oom_moe_tiled_nvfp4");
     }
-    if (k % TW_BK == 0 && w_off % 16 == 0 && s_off % 2 == 0) {
-        // 640-row tiles, weights straight into registers (records' parts are 16-byte aligned
-        // in the released layout)
+    if (route == TiledRoute::wide) {
         const dim3 grid((unsigned)cdiv(n, TW_BN), (unsigned)cdiv(max_per_expert, TW_BM), (unsigned)n_experts);
         if (precision == OOM_EXPERT_EXACT)
             hipLaunchKernelGGL(moe_tiled_nvfp4_wide_kernel<3>, grid, dim3(TW_THREADS), 0, as_stream(stream), a);

@@ -970,38 +970,6 @@ static bool kv_row_shape(int d, int bits) {
     return d >= 32 && d % 32 == 0 && d <= TQ_MAXD && (bits == 0 || ((d & (d - 1)) == 0 && bits >= 2 && bits <= 8));
 }
 
-// How a KV head's keys are dealt: blocks of `waves` waves, `blocks` of them a KV head. A wave's
-// groups follow each other (about 4 us each: 128 fp32 MFMAs and the decoding between them), so
-// every wave takes one group as long as the grid then has a block a CU or fewer:
-//   - blocks of 4 waves, one a SIMD, while ceil(groups / 4) blocks a KV head make at most
-//     TT_FILL in all; past that two of them share a CU (9001 keys, 2 KV heads, us a call with
-//     the combine: 27.7 as 282 blocks of 4 waves, 18.7 as 142 of 8);
-//   - else blocks of 8 waves, at most TT_FILL in all, their waves taking more groups from there;
-//   - fp32 rows (no decoding for a second wave's MFMAs to hide behind) keep 4 waves up to two
-//     groups a wave: 17.0 us against 19.4 at 9001 keys, 2 KV heads.
-// Before, every wave was sized for two groups on blocks of 8: us a call then and now, k8v6, all
-// keys visible, 2 KV heads: 24.4 -> 15.5 at 700 keys, 24.5 -> 16.1 at 4500, 24.7 -> 18.7 at
-// 9001, 24.8 -> 19.8 at 16384, 26.2 at 32768 (the same split).
-constexpr int TT_FILL = 256;
-
-struct TurboSplit {
-    int waves, blocks;
-};
-
-static TurboSplit turbo_split(int kv_len, int kv_heads, bool fp32) {
-    const int groups = (kv_len + 15) / 16, most = std::max(1, TT_FILL / kv_heads);
-    for (int per = 4; per <= (fp32 ? 8 : 4); per += 4)
-        if ((groups + per - 1) / per <= most) return {4, (groups + per - 1) / per};
-    return {8, std::min((groups + 7) / 8, most)};
-}
-
-// Two groups a wave on blocks of 8 waves: the fewest partials, for a workspace with room for
-// no more.
-static TurboSplit turbo_split_least(int kv_len, int kv_heads) {
-    const int groups = (kv_len + 15) / 16;
-    return {8, std::max(1, std::min((groups + 15) / 16, std::max(1, TT_FILL / kv_heads)))};
-}
-
 static size_t t_al256(size_t v) { return (v + 255) & ~size_t(255); }
 
 // Offset of the maxima and sums behind the partial outputs, and the bytes of both.

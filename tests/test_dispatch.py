@@ -1,0 +1,28 @@
+"""The host rules that pick a kernel or a split (homelab_amd/csrc/dispatch.hpp), on the CPU."""
+import pytest
+
+import dispatch
+
+
+@pytest.mark.parametrize("n,k,w_off,s_off,e,max_n,exact,want", [
+    (640, 2560, 256, 819456, 512, 20, True, "rows"),   # the released record's gate, ten rows an expert
+    (2560, 640, 256, 819456, 512, 20, False, "rows"),  # and its down
+    (640, 4096, 256, 819456, 512, 20, True, "wide"),   # K past eight slices of ten steps
+    (640, 2592, 256, 819456, 512, 20, True, "narrow"),  # K no whole K block
+    (640, 2560, 258, 819456, 512, 20, True, "narrow"),  # codes at 2 bytes of alignment
+    (640, 2560, 260, 819456, 512, 20, True, "rows"),
+])
+def test_tiled_route(n, k, w_off, s_off, e, max_n, exact, want):
+    assert dispatch.tiled(n, k, w_off, s_off, e, max_n, exact) == want
+
+
+def test_turbo_split_covers_the_keys():
+    """Every split deals every group of 16 keys, on at most 256 blocks over the KV heads, and one
+    block a KV head past 256 of them."""
+    shapes = [(n, h, f) for n in range(1, 70000, 487) for h in (1, 2, 3, 4, 7, 8, 64, 256, 300) for f in (0, 1)]
+    for (n, h, f), ans in zip(shapes, dispatch.ask(*(f"turbo {n} {h} {f}" for n, h, f in shapes))):
+        waves, blocks = map(int, ans.split())
+        groups = -(-n // 16)
+        assert waves in (4, 8) and 1 <= blocks and (blocks == 1 or blocks * h <= 256)
+        assert (blocks - 1) * waves < groups, "an empty block"
+        assert waves == 8 or blocks * waves * (2 if f else 1) >= groups
