@@ -82,14 +82,17 @@ constexpr int64_t N4S_XMAX = 144 * 1024; // of LDS for the tokens' x, beside the
 // assignments can reach) to pay for staging all of x in every block. The whole step, staged
 // against this: 64 experts of 1040 / 272 (18 M) 35.6 and 38.3 us, 8 of 1024 / 256 (2 M) 20.0
 // and 20.9; 20 of 2560 / 640 (33 M) 40.4 and 40.0, 80 (131 M) 97 and 86, 144 of 2560 / 1536
-// (566 M) 113 and 95.
+// (566 M) 113 and 95. At most three chunks of 1024 columns: with four the two rounds of loads in
+// flight spill 79 registers (512 experts top-10, 4096 / 1536: 64 us staged and 94 at 2 tokens, 243
+// and 325 at 8; 128 top-8, 4096 / 768: 104 and 142 at 8).
+constexpr int64_t N4S_MAX_H = 3072;
 constexpr int64_t N4S_MIN_ROWS = 24ll << 20;  // experts x hidden x inter
 inline int64_t gate_up_step_lds(int T, int64_t hidden) {
     return (T + 1) / 2 * 2 * cdiv(hidden, 1024) * 4096;  // staged two rows at a time
 }
 inline bool gate_up_step_ok(int T, int E, int k, int64_t hidden, int64_t inter) {
     const int64_t A = (int64_t)T * k;
-    return A <= N4S_AMAX && gate_up_step_lds(T, hidden) <= N4S_XMAX &&
+    return A <= N4S_AMAX && hidden <= N4S_MAX_H && gate_up_step_lds(T, hidden) <= N4S_XMAX &&
            std::min<int64_t>(E, A) * hidden * inter >= N4S_MIN_ROWS;
 }
 

@@ -987,8 +987,7 @@ static int launch_gate_up_step(const uint64_t* recs, const PlanView& pv, const v
     return xdt == OOM_BF16 ? launch_gate_up_step_t<OOM_BF16, C>(recs, pv, x, T, h, geo, st)             \
                            : launch_gate_up_step_t<OOM_F32, C>(recs, pv, x, T, h, geo, st);
     if (ch <= 2) { N4S_CASE(2) }
-    if (ch == 3) { N4S_CASE(3) }
-    N4S_CASE(4)
+    N4S_CASE(3)
 #undef N4S_CASE
 }
 

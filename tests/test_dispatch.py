@@ -16,6 +16,18 @@ def test_tiled_route(n, k, w_off, s_off, e, max_n, exact, want):
     assert dispatch.tiled(n, k, w_off, s_off, e, max_n, exact) == want
 
 
+@pytest.mark.parametrize("T,E,k,hidden,inter,want", [
+    (8, 512, 10, 2560, 640, "step"),
+    (8, 512, 10, 3072, 1024, "step"),
+    # past three chunks of 1024 the kernel's two rounds of loads spill
+    (2, 512, 10, 4096, 1536, "staged"),
+    (8, 128, 8, 4096, 768, "staged"),
+    (4, 64, 8, 3088, 1536, "staged"),
+])
+def test_step_route(T, E, k, hidden, inter, want):
+    assert dispatch.step(T, E, k, hidden, inter) == want
+
+
 def test_turbo_split_covers_the_keys():
     """Every split deals every group of 16 keys, on at most 256 blocks over the KV heads, and one
     block a KV head past 256 of them."""
