@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 
 namespace oom {
 
@@ -78,22 +79,36 @@ inline TiledRoute tiled_route(int64_t N, int64_t K, int64_t w_off, int64_t s_off
 constexpr int N4S_AMAX = 512;            // assignments of a step (and so routed experts)
 constexpr int64_t N4S_XMAX = 144 * 1024; // of LDS for the tokens' x, beside the plan's 12 KiB
 
-// A step whose tokens' x fits LDS beside the plan, with rows enough (the most that its
-// assignments can reach) to pay for staging all of x in every block. The whole step, staged
-// against this: 64 experts of 1040 / 272 (18 M) 35.6 and 38.3 us, 8 of 1024 / 256 (2 M) 20.0
-// and 20.9; 20 of 2560 / 640 (33 M) 40.4 and 40.0, 80 (131 M) 97 and 86, 144 of 2560 / 1536
-// (566 M) 113 and 95. At most three chunks of 1024 columns: with four the two rounds of loads in
-// flight spill 79 registers (512 experts top-10, 4096 / 1536: 64 us staged and 94 at 2 tokens, 243
-// and 325 at 8; 128 top-8, 4096 / 768: 104 and 142 at 8).
+// Whether a step's gate/up runs as free-running waves over all its tokens' x, instead of staged
+// per expert (the same bits). The plan and x fit LDS; at most three chunks of 1024 columns: with
+// four the two rounds of loads in flight spill 79 registers (512 experts top-10, 4096 / 1536: 64
+// us staged and 94 at 2 tokens, 243 and 325 at 8; 128 top-8, 4096 / 768: 104 and 142 at 8).
+// And rows enough: every block stages all of x before its first sums, a wave's last round of
+// items leaves others idle, and a row is decoded once an assignment where the staged launch
+// decodes it once for two. So the rule is on the items a wave, of four rows of a routed expert,
+// with the experts that evenly spread picks reach. Us a step, staged and this, by items a wave
+// and assignments an expert:
+//   three chunks (2560 / 640): 1.2, 2.1: 33.6, 36.7 (4 tokens, 16 experts top-8); 1.55, 1.0: 33.9,
+//     35.1 (2, 512 top-10); 3.3, 1.5: 57.8, 58.8 (8, 64 top-8); 3.0, 1.0: 53.3, 48.9 (4, 512
+//     top-10); 3.7, 1.7: 66.6, 65.7 (8, 64 top-10); 5.8, 1.1: 92.9, 82.6 (8, 512 top-10)
+//   two (2048 / 1024): 1.7, 1.1: 27.5, 28.6; 2.7, 1.5: 35.9, 36.9; 3.9, 3.1: 67.4, 69.6; 4.4, 1.4:
+//     47.8, 46.0; 6.3, 1.9: 84.2, 78.5; 10.3, 1.6: 118, 103
+//   one (1024 / 512), where the decoding weighs most: 2.0, 6.0: 57.3, 61.5; 4.0, 4.1: 67.6, 72.2;
+//     5.2, 1.6: 50.9, 50.9; 7.0, 2.3: 69.9, 74.0; 8.7, 1.2: 70.1, 66.6; 15, 1.3: 115, 108
 constexpr int64_t N4S_MAX_H = 3072;
-constexpr int64_t N4S_MIN_ROWS = 24ll << 20;  // experts x hidden x inter
+constexpr int N4S_WAVES = 8;    // waves a block, on one block a CU
+constexpr int N4S_GRID = 256;
+constexpr int N4S_ROWS = 4;     // gate (and up) rows an item
 inline int64_t gate_up_step_lds(int T, int64_t hidden) {
     return (T + 1) / 2 * 2 * cdiv(hidden, 1024) * 4096;  // staged two rows at a time
 }
 inline bool gate_up_step_ok(int T, int E, int k, int64_t hidden, int64_t inter) {
     const int64_t A = (int64_t)T * k;
-    return A <= N4S_AMAX && hidden <= N4S_MAX_H && gate_up_step_lds(T, hidden) <= N4S_XMAX &&
-           std::min<int64_t>(E, A) * hidden * inter >= N4S_MIN_ROWS;
+    if (A > N4S_AMAX || hidden > N4S_MAX_H || gate_up_step_lds(T, hidden) > N4S_XMAX) return false;
+    const double experts = E * (1.0 - std::pow(1.0 - (double)k / E, T));
+    const double items = experts * (double)cdiv(inter, N4S_ROWS) / (N4S_GRID * N4S_WAVES), per = A / experts;
+    if (hidden <= 1024) return items >= (per <= 1.75 ? 5.0 : 8.0);
+    return items >= (per <= 1.1 ? 2.9 : hidden <= 2048 ? 4.0 : 3.5);
 }
 
 // ---- oom_attn_decode_turbo (turbo.hip) ------------------------------------------------------

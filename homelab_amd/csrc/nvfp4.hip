@@ -523,7 +523,7 @@ __device__ __forceinline__ void dn4_compute(const Dn4W& w, const float4* xs4, co
 // one's sums: 40 us there, bound by the conversions and sums of the assignments. The
 // arithmetic is gu4_math's, so every output has the staged kernel's bits. Down stays staged:
 // the same form of it re-reads an expert's h per wave and took 39 us against 30.
-constexpr int N4S_WAVES = 8;
+static_assert(N4S_ROWS == 2 * N4_GP, "an item is a gate/up pass of a wave");
 
 // The step's plan as the waves read it.
 struct Plan4Lds {
@@ -975,7 +975,7 @@ static int launch_gate_up_step_t(const uint64_t* recs, const PlanView& pv, const
             return fail(OOM_ERR_LAUNCH, "oom_moe_decode_nvfp4: the device refused the step's LDS");
         raised_dev = dev;
     }
-    hipLaunchKernelGGL((moe_gate_up_nvfp4_step_kernel<XDT, CS>), dim3(256), dim3(64 * N4S_WAVES), lds, st, recs, pv.off(),
+    hipLaunchKernelGGL((moe_gate_up_nvfp4_step_kernel<XDT, CS>), dim3(N4S_GRID), dim3(64 * N4S_WAVES), lds, st, recs, pv.off(),
                        pv.assign_tok(), x, T, h, rec4_of(geo), pv.n_e());
     return launched("moe_gate_up_nvfp4");
 }

@@ -23,6 +23,23 @@ def test_tiled_route(n, k, w_off, s_off, e, max_n, exact, want):
     (2, 512, 10, 4096, 1536, "staged"),
     (8, 128, 8, 4096, 768, "staged"),
     (4, 64, 8, 3088, 1536, "staged"),
+    # few rounds of items a wave: a step's experts x rows / 4 over 2048 waves
+    (2, 512, 10, 2560, 640, "staged"),
+    (2, 128, 8, 2560, 640, "staged"),
+    (4, 512, 10, 2560, 640, "step"),
+    (4, 16, 8, 2560, 640, "staged"),
+    # several assignments an expert, which the step decodes a row for each and the staged launch in pairs
+    (8, 16, 8, 2560, 640, "staged"),
+    (8, 64, 8, 2560, 640, "staged"),
+    (24, 128, 8, 1024, 512, "staged"),
+    (32, 64, 8, 1024, 512, "staged"),
+    (32, 512, 10, 1024, 512, "step"),
+    (16, 128, 8, 2048, 1536, "step"),
+    (16, 64, 8, 2048, 1536, "step"),
+    # past the plan's 512 slots; x past its LDS
+    (33, 128, 16, 1008, 304, "staged"),
+    (13, 512, 10, 2560, 640, "staged"),
+    (12, 512, 10, 2560, 640, "step"),
 ])
 def test_step_route(T, E, k, hidden, inter, want):
     assert dispatch.step(T, E, k, hidden, inter) == want
