@@ -8,6 +8,12 @@
 #include <algorithm>
 #include <cmath>
 
+#ifdef __HIPCC__
+#define OOM_HD __host__ __device__  // the device asks some of it too
+#else
+#define OOM_HD
+#endif
+
 namespace oom {
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -35,7 +41,8 @@ struct RowsSplit {
 inline RowsSplit rows_split(int64_t K) {
     RowsSplit s{0, 10};
     while (s.ks_log < 3 && K > (int64_t)320 << s.ks_log) s.ks_log++;
-    s.st = std::max(6, 2 * (int)cdiv(K, (int64_t)64 << s.ks_log));
+    s.st = 2 * (int)cdiv(K, (int64_t)64 << s.ks_log);
+    if (s.st < 6) s.st = 6;
     return s;
 }
 // Batches of weight rows that a projection of N rows has.
@@ -43,35 +50,133 @@ inline int rows_batches(int64_t N, const RowsSplit& sp) {
     return (int)cdiv(N, 16 * NR_BATCH * (NR_WAVES >> sp.ks_log));
 }
 
-// Where the rows kernel is the better one: K in whole scale groups a lane and at most 8 slices
-// of 10 steps, and either slices and batches that K and N fill (five sixths at least) or tiles
-// of so few rows that the stream counts and not the steps. Us a call of gate, up, SwiGLU, down
-// and combine at 2560 / 640, exact, rows kernel and tiles: 512 experts top-10, 60 tokens 287
-// and 601, 250 398 and 698, 500 451 and 722, 900 664 and 761, 1050 766 and 782, 1400 924 and
-// 1224, 2048 1218 and 1472; 64 experts, 300 tokens 228 and 296, 1200 612 and 626. At 1600 / 448
-// (slices 78 % and 88 % full) 128 experts top-4, 600 tokens 151 and 185, but 64 experts top-10,
-// 1200 tokens (190 rows an expert) 398 and 327. The tiles also keep the steps of many experts
-// whose 41 to 48 rows at most are one 48-row tile where the rows kernel decodes twice or more
-// (512 experts, 1200 tokens: 815 and 786; with 128 experts 264 and 299).
-inline bool rows_kernel_serves(int64_t N, int64_t K, int64_t w_off, int64_t s_off, int64_t n_experts, int64_t max_n,
-                               bool exact) {
-    if (K % 64 != 0 || K > NR_MAXK || w_off % 4 != 0 || s_off % 4 != 0) return false;
-    const RowsSplit sp = rows_split(K);
-    if (n_experts * cdiv(max_n, NR_M) * rows_batches(N, sp) > INT32_MAX) return false;
-    if (exact && K % TW_BK == 0 && n_experts >= 384 && max_n > 40 && max_n <= TW_BM) return false;
-    const int64_t rows = (int64_t)16 * NR_BATCH * (NR_WAVES >> sp.ks_log) * rows_batches(N, sp);
-    return 6 * K * N >= 5 * ((int64_t)32 * sp.st << sp.ks_log) * rows || max_n <= 48;
+// The tiles kernel of a shape: wide tiles where the weights can go straight into registers
+// (records' parts are 16-byte aligned in the released layout).
+inline bool tiled_wide(int64_t K, int64_t w_off, int64_t s_off) {
+    return K % TW_BK == 0 && w_off % 16 == 0 && s_off % 2 == 0;
 }
 
-enum class TiledRoute { rows, wide, narrow };
+// What the few-row kernel can serve at all: K in whole scale groups a lane and at most 8 slices
+// of 10 steps.
+inline bool rows_kernel_serves(int64_t N, int64_t K, int64_t w_off, int64_t s_off, int64_t n_experts, int64_t max_n) {
+    return K % 64 == 0 && K <= NR_MAXK && w_off % 4 == 0 && s_off % 4 == 0 &&
+           n_experts * cdiv(max_n, NR_M) * rows_batches(N, rows_split(K)) <= INT32_MAX / 8;
+}
 
-// The kernel of a projection of N rows of K inputs over n_experts experts of at most max_n
-// assignments.
+// Blocks that each XCD gets: workgroup i of a launch runs on XCD i % 8.
+struct XcdBlocks {
+    int32_t on[8] = {};
+    // `times` runs of n workgroups from workgroup `first` on
+    OOM_HD void add(uint32_t first, int32_t n, int32_t times = 1) {
+        for (uint32_t i = 0; i < 8; i++) on[i] += times * (n / 8 + (((i - first) & 7) < (uint32_t)n % 8 ? 1 : 0));
+    }
+};
+
+// The tiles kernel's launch: workgroup x + nx (y + ny e) is N tile x, assignment tile y of expert e,
+// and ends at once where expert e has no such tile.
+struct TiledGrid {
+    int32_t nx, ny, rows;  // rows: assignments a tile
+};
+inline TiledGrid tiled_grid(int64_t N, int64_t max_n, bool wide) {
+    const int32_t bn = wide ? TW_BN : T4_BN, bm = wide ? TW_BM : T4_BM;
+    return {(int32_t)cdiv(N, bn), (int32_t)cdiv(max_n, bm), bm};
+}
+
+// What a projection takes by either kernel, in ns, by what its experts' assignments make of it:
+// t16 tiles of 16 for the few-row kernel, whose blocks take equal runs of the tiles' batches and load
+// a new tile's activations; rounds of one block a CU on the busiest XCD for the wide tiles; blocks
+// in flight together for the narrow ones. In whole numbers, so that every place that asks gets one
+// answer. Fitted to 4500 calls (N 256 to 4096, K 320 to 2560, 4 to 512 experts, 1 to 900 rows an
+// expert, even and skewed): half of them within 5 % of what they took, nine tenths within 20 %.
+struct TiledCost {
+    int32_t start, batch, tile, batches;  // few-row kernel
+    int32_t once, round;                  // tiles
+    bool wide;
+    OOM_HD int64_t rows_ns(int32_t t16) const {
+        return start + batch * (((int64_t)t16 * batches + 255) >> 8) + ((int64_t)tile * t16 >> 8);
+    }
+    OOM_HD int64_t tiles_ns(const XcdBlocks& blocks) const {
+        int32_t most = 0;
+        for (int i = 0; i < 8; i++) most = blocks.on[i] > most ? blocks.on[i] : most;
+        return once + (wide ? (int64_t)round * ((most + 31) >> 5) : (int64_t)round * (most > 32 ? most : 32) >> 5);
+    }
+    OOM_HD bool rows_faster(int32_t t16, const XcdBlocks& blocks) const { return rows_ns(t16) <= tiles_ns(blocks); }
+};
+inline TiledCost tiled_cost(int64_t N, int64_t K, bool wide, bool exact) {
+    const RowsSplit sp = rows_split(K);
+    TiledCost c;
+    c.batches = rows_batches(N, sp);
+    const int i = sp.st == 6 ? 0 : sp.st == 8 ? 1 : 2;
+    const int32_t rows[2][3][3] = {{{5600, 5560, 3800}, {6400, 6860, 4800}, {6900, 8900, 5600}},
+                                   {{5600, 6880, 3800}, {6600, 8340, 5000}, {9600, 11000, 6300}}};
+    c.start = rows[exact][i][0], c.batch = rows[exact][i][1], c.tile = rows[exact][i][2];
+    const int32_t k = (int32_t)K;
+    if (wide) {  // waves past N are idle: of the round's time per column, a part goes with the rows there are
+        const int32_t full = (int32_t)(k * N / (TW_BN * cdiv(N, TW_BN)));
+        c.once = exact ? -75 * k / 10 : -69 * k / 10;
+        c.round = exact ? 5050 + (345 * k + 87 * full) / 10 : 3900 + (202 * k + 122 * full) / 10;
+    } else {
+        c.once = exact ? 68 * k / 10 : 29 * k / 10;
+        c.round = exact ? 190 + 162 * k / 10 : 146 * k / 10 - 390;
+    }
+    c.wide = wide;
+    return c;
+}
+
+// The kernels that a call launches: the few-row kernel (rows), the tiles (wide or narrow), or both,
+// which then count the assignments on the device: one of them works, the other returns at once.
+struct TiledRoute {
+    bool rows, tiles, wide;
+};
+
+// The host knows the largest expert only. Evenly spread picks reach it with most experts near it,
+// and then the tiles are the faster ones, up to twice, once experts fill them (us a projection,
+// exact, few-row kernel and tiles: 640 x 2560, 64 experts, 320 rows each, 295 and 251; 2560 x 640,
+// 32 experts, 75 rows each, 60 and 36). Skewed picks reach it with most experts far below, and the
+// few-row kernel is the faster one, up to three times: the tiles pad to 48 or 64, and the experts'
+// first tiles alone can fall on half of the XCDs. So: the few-row kernel where it is the faster one
+// of evenly spread picks, the tiles where they are with every expert but one in a single tile, both
+// between the two. The second launch and the counting cost 3.3 us and 1 us a round of tiles, so a
+// call whose tiles take less than TR_COUNT_NS takes one kernel alone, as does one whose evenly spread
+// picks make a twentieth of difference, one with more experts than a block counts in a few loads, or
+// one with sums past 2^24 (the device's are f32).
+constexpr int64_t TR_COUNT_NS = 50000;
+constexpr int TR_COUNT_E = 2048;
 inline TiledRoute tiled_route(int64_t N, int64_t K, int64_t w_off, int64_t s_off, int64_t n_experts, int64_t max_n,
                               bool exact) {
-    if (rows_kernel_serves(N, K, w_off, s_off, n_experts, max_n, exact)) return TiledRoute::rows;
-    // weights straight into registers (records' parts are 16-byte aligned in the released layout)
-    return K % TW_BK == 0 && w_off % 16 == 0 && s_off % 2 == 0 ? TiledRoute::wide : TiledRoute::narrow;
+    const bool wide = tiled_wide(K, w_off, s_off);
+    if (!rows_kernel_serves(N, K, w_off, s_off, n_experts, max_n)) return {false, true, wide};
+    const TiledGrid grid = tiled_grid(N, max_n, wide);
+    const TiledCost cost = tiled_cost(N, K, wide, exact);
+    // the blocks if each expert has `lo` tiles and `hi` of them one more, both spread evenly
+    const auto blocks = [&](int64_t lo, int64_t hi) {
+        XcdBlocks b;
+        for (int j = 0; j < 8; j++) {  // the experts e with e % 8 == j start on one XCD
+            const int64_t n = (n_experts + 7 - j) / 8, m = std::min(n, (hi + 7 - j) / 8);
+            const uint32_t first = (uint32_t)grid.nx * grid.ny * j;
+            b.add(first, (int32_t)(grid.nx * lo), (int32_t)n);
+            b.add(first + (uint32_t)(grid.nx * lo), grid.nx, (int32_t)m);
+        }
+        return b;
+    };
+    // mean rows of evenly spread picks whose largest expert has max_n: sqrt(2 mean ln E) below it
+    const double spread = 2.0 * std::log((double)std::max<int64_t>(n_experts, 2));
+    const double root = (std::sqrt(spread + 4.0 * (double)max_n) - std::sqrt(spread)) / 2.0;
+    const double mean = std::max(1.0, root * root);
+    const auto tiles = [&](int64_t m) {
+        return std::min(n_experts * cdiv(max_n, m), (int64_t)((double)n_experts * std::max(1.0, mean / (double)m + 0.5)));
+    };
+    const int64_t t16 = tiles(NR_M), tn = tiles(grid.rows);
+    const XcdBlocks even = blocks(tn / n_experts, tn % n_experts);
+    const int64_t ns = cost.tiles_ns(even);
+    if (cost.rows_ns((int32_t)t16) <= ns + (ns < TR_COUNT_NS ? 0 : ns / 20)) return {true, false, wide};
+    XcdBlocks skewed = blocks(1, 0);
+    skewed.add(0, grid.nx * (grid.ny - 1));
+    const int64_t sums = n_experts * std::max(cdiv(max_n, NR_M), (int64_t)grid.nx * grid.ny);
+    if (n_experts > TR_COUNT_E || sums >= 1 << 24 || ns < TR_COUNT_NS ||
+        !cost.rows_faster((int32_t)(cdiv(max_n, NR_M) + n_experts - 1), skewed))
+        return {false, true, wide};
+    return {true, true, wide};
 }
 
 // ---- oom_moe_decode_nvfp4, several tokens (nvfp4.hip) -------------------------------------

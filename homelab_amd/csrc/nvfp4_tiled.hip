@@ -44,7 +44,41 @@ struct TiledArgs {
     int N, K;
     int64_t w_off, s_off;  // the projection's codes and e4m3 scales in a record
     int s2_idx;            // its weight_scale_2, in floats from the record start
+    int n_experts, max_n;  // experts, and assignments of the largest
+    bool counted;          // both kernels are launched
+    TiledGrid grid;        // of the tiles kernel
+    TiledCost cost;
 };
+
+// Whether the few-row kernel is the faster one for this call's assignments. Every block of both
+// kernels counts them, so exactly one of the two works. (The sums are whole
+// numbers below 2^24: exact in f32.)
+template <int WAVES>
+__device__ __forceinline__ bool counted_rows_faster(const TiledArgs& g) {
+    __shared__ float part[16][WAVES];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int t16 = 0;
+    XcdBlocks blocks;
+    for (int e = threadIdx.x; e < g.n_experts; e += 64 * WAVES) {
+        const int n = min(max(g.off[e + 1] - g.off[e], 0), g.max_n);
+        t16 += (n + NR_M - 1) / NR_M;
+        const int tiles = g.grid.rows == TW_BM ? (n + TW_BM - 1) / TW_BM : (n + T4_BM - 1) / T4_BM;
+        blocks.add((unsigned)g.grid.nx * g.grid.ny * e, g.grid.nx * tiles);
+    }
+    float v[16] = {};
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = (float)blocks.on[i];
+    v[8] = (float)t16;
+    const float sum = wave_sum_multi<16>(v, lane);  // v[i] on lane 4 i
+    if ((lane & 3) == 0) part[lane >> 2][wave] = sum;
+    __syncthreads();
+    float s = 0.0f;
+    for (int w = 0; w < WAVES; w++) s += part[lane & 15][w];
+    const auto total = [&](int i) { return __builtin_amdgcn_readlane((int)s, i); };
+#pragma unroll
+    for (int i = 0; i < 8; i++) blocks.on[i] = total(i);
+    return g.cost.rows_faster(total(8), blocks);
+}
 
 typedef __bf16 t4bf16x2 __attribute__((ext_vector_type(2)));
 typedef float t4f32x2 __attribute__((ext_vector_type(2)));
@@ -63,6 +97,7 @@ __global__ void __launch_bounds__(T4_THREADS, 2) moe_tiled_nvfp4_kernel(TiledArg
     const int e = blockIdx.z;
     const int a_begin = g.off[e] + (int)blockIdx.y * T4_BM, a_end = g.off[e + 1];
     if (a_begin >= a_end) return;
+    if (g.counted && counted_rows_faster<T4_THREADS / 64>(g)) return;
     const int nt = min(T4_BM, a_end - a_begin);
     const int r0 = (int)blockIdx.x * T4_BN;
     const uint8_t* rec = reinterpret_cast<const uint8_t*>(g.recs[e]);
@@ -209,21 +244,26 @@ __global__ void __launch_bounds__(T4_THREADS, 2) moe_tiled_nvfp4_kernel(TiledArg
 
 // ---- wide tiles: all 640 rows of a projection tile over 48 assignments ---------------
 //
-// For K past the few-row kernel's slices, or where rows_kernel_serves finds these the better.
+// For K past the few-row kernel's slices, or where these are the faster (tiled_route).
 // The 128-row tiles above gather every activation row once per N tile, four times the
 // bytes of the weights they meet. Here a block of 8 waves takes 640 weight rows (wave w:
-// rows 80 w .. + 80, five 16-row N subtiles) x 64 assignments, so a gate or up projection
+// rows 80 w .. + 80, five 16-row N subtiles) x 48 assignments, so a gate or up projection
 // (N 640) gathers each activation row once. The weights never pass through LDS: lane
 // (r, q) of a wave (r = lane % 16, q = lane / 16) loads 16 contiguous code bytes of its row
 // per K block of 128, codes k = 32 q .. 32 q + 31 of the block, and feeds them to four
 // MFMAs, codes 8 s .. 8 s + 7 at step s. The activations sit in LDS in the same order
 // (the lane's A operand at step s is x[m][32 q + 8 s .. + 8]), so every product pairs the
 // same k on both sides and the sum is the plain dot product. Per K block the block loads
-// 64 x 128 fp32 activations (four 16-byte loads a thread) while the previous block runs,
+// 48 x 128 fp32 activations (three 16-byte loads a thread) while the previous block runs,
 // splits them into their bf16 terms in LDS (row stride 272 bytes: the 16 rows of an
 // operand read fall in distinct bank groups), and each wave decodes its own weights in
 // registers: e2m1 -> f32 (v_cvt_scalef32_pk_f32_fp4 at scale 1), times the e4m3 group
 // scale, -> bf16 (exact, as above). K must be a multiple of 128.
+// Workgroups go to the XCDs in the grid's order (N tile, assignment tile, expert), so where the
+// tiles an expert could have make an even number of workgroups and most experts have one, half of
+// the XCDs get little. An odd number of assignment tiles mends that (0.5 to 0.97 of the time for
+// skewed picks) but takes 1.2 to 1.7 of it where even ones put one block on each CU, so the grid is
+// as it is and tiled_route counts the blocks per XCD.
 constexpr int TW_NS = 5;         // N subtiles a wave
 constexpr int TW_THREADS = 512;  // 8 waves
 constexpr int TW_LS = 136;       // LDS row stride in bf16 (272 bytes)
@@ -235,6 +275,7 @@ __global__ void __launch_bounds__(TW_THREADS) moe_tiled_nvfp4_wide_kernel(TiledA
     const int e = blockIdx.z;
     const int a_begin = g.off[e] + (int)blockIdx.y * TW_BM, a_end = g.off[e + 1];
     if (a_begin >= a_end) return;
+    if (g.counted && counted_rows_faster<TW_THREADS / 64>(g)) return;
     const int nt = min(TW_BM, a_end - a_begin);
     const int r0 = (int)blockIdx.x * TW_BN;
     const uint8_t* rec = reinterpret_cast<const uint8_t*>(g.recs[e]);
@@ -387,14 +428,15 @@ __global__ void __launch_bounds__(TW_THREADS) moe_tiled_nvfp4_wide_kernel(TiledA
 constexpr int TR_LIST = 1024;  // tiles a block can have
 
 template <int TERMS, int ST>
-__global__ void __launch_bounds__(64 * NR_WAVES) moe_tiled_nvfp4_rows_kernel(TiledArgs g, int n_experts, int max_n,
-                                                                            int batches, int ks_log) {
+__global__ void __launch_bounds__(64 * NR_WAVES) moe_tiled_nvfp4_rows_kernel(TiledArgs g, int batches, int ks_log) {
     __shared__ RowsLds lds;
     __shared__ int2 list[TR_LIST];
     __shared__ int wtot[NR_WAVES];
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ks = 1 << ks_log, slice = wave & (ks - 1), group = wave >> ks_log, ngroups = NR_WAVES >> ks_log;
+    if (g.counted && !counted_rows_faster<NR_WAVES>(g)) return;
+    const int n_experts = g.n_experts, max_n = g.max_n;
     // ---- the block's share of the tiles' batches: tiles counted in expert order
     const int per = (n_experts + 64 * NR_WAVES - 1) / (64 * NR_WAVES);
     const int e0 = min(n_experts, tid * per), e1 = min(n_experts, e0 + per);
@@ -486,26 +528,33 @@ __global__ void __launch_bounds__(64 * NR_WAVES) moe_tiled_nvfp4_rows_kernel(Til
 }
 
 template <int TERMS>
-static void launch_tiled_rows(const TiledArgs& a, int n_experts, int max_per_expert, hipStream_t st) {
+static void launch_tiled_rows(const TiledArgs& a, hipStream_t st) {
     const RowsSplit sp = rows_split(a.K);
     const int batches = rows_batches(a.N, sp);
-    const int64_t most = (int64_t)n_experts * cdiv(max_per_expert, NR_M);  // tiles
+    const int64_t most = (int64_t)a.n_experts * cdiv(a.max_n, NR_M);  // tiles
     const dim3 grid((unsigned)std::max(std::min<int64_t>(256, most * batches), cdiv(most, TR_LIST - 2)));
-    const dim3 block(64 * NR_WAVES);
-    switch (sp.st) {
-        case 6:
-            hipLaunchKernelGGL((moe_tiled_nvfp4_rows_kernel<TERMS, 6>), grid, block, 0, st, a, n_experts,
-                               max_per_expert, batches, sp.ks_log);
-            break;
-        case 8:
-            hipLaunchKernelGGL((moe_tiled_nvfp4_rows_kernel<TERMS, 8>), grid, block, 0, st, a, n_experts,
-                               max_per_expert, batches, sp.ks_log);
-            break;
-        default:
-            hipLaunchKernelGGL((moe_tiled_nvfp4_rows_kernel<TERMS, 10>), grid, block, 0, st, a, n_experts,
-                               max_per_expert, batches, sp.ks_log);
-            break;
+    const auto kernel = sp.st == 6   ? moe_tiled_nvfp4_rows_kernel<TERMS, 6>
+                        : sp.st == 8 ? moe_tiled_nvfp4_rows_kernel<TERMS, 8>
+                                     : moe_tiled_nvfp4_rows_kernel<TERMS, 10>;
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * NR_WAVES), 0, st, a, batches, sp.ks_log);
+}
+
+template <int TERMS>
+static void launch_tiled_tiles(const TiledArgs& a, bool wide, hipStream_t st) {
+    const dim3 grid((unsigned)a.grid.nx, (unsigned)a.grid.ny, (unsigned)a.n_experts);
+    if (wide) hipLaunchKernelGGL(moe_tiled_nvfp4_wide_kernel<TERMS>, grid, dim3(TW_THREADS), 0, st, a);
+    else hipLaunchKernelGGL(moe_tiled_nvfp4_kernel<TERMS>, grid, dim3(T4_THREADS), 0, st, a);
+}
+
+template <int TERMS>
+static int launch_tiled(const TiledArgs& a, const TiledRoute& route, hipStream_t st) {
+    if (route.rows) {
+        launch_tiled_rows<TERMS>(a, st);
+        if (int rc = launched("oom_moe_tiled_nvfp4")) return rc;
     }
+    if (!route.tiles) return OOM_OK;
+    launch_tiled_tiles<TERMS>(a, route.wide, st);
+    return launched("oom_moe_tiled_nvfp4");
 }
 
 __global__ void __launch_bounds__(256) moe_swiglu_kernel(const float* __restrict__ gt, const float* __restrict__ up,
@@ -531,27 +580,13 @@ extern "C" int oom_moe_tiled_nvfp4(const uint64_t* recs, const int32_t* off, con
     if (n_experts == 0 || max_per_expert == 0) return OOM_OK;
     OOM_REQUIRE(recs && off && x && y, "oom_moe_tiled_nvfp4: null buffer");
     OOM_REQUIRE(aligned(x, 16), "oom_moe_tiled_nvfp4: x must be 16-byte aligned");
-    TiledArgs a{recs, off, rows, x, y, n, k, w_off, s_off, s2_idx};
-    const TiledRoute route = tiled_route(n, k, w_off, s_off, n_experts, max_per_expert, precision == OOM_EXPERT_EXACT);
-    if (route == TiledRoute::rows) {
-        if (precision == OOM_EXPERT_EXACT) launch_tiled_rows<3>(a, n_experts, max_per_expert, as_stream(stream));
-        else launch_tiled_rows<1>(a, n_experts, max_per_expert, as_stream(stream));
-        return launched("oom_moe_tiled_nvfp4");
-    }
-    if (route == TiledRoute::wide) {
-        const dim3 grid((unsigned)cdiv(n, TW_BN), (unsigned)cdiv(max_per_expert, TW_BM), (unsigned)n_experts);
-        if (precision == OOM_EXPERT_EXACT)
-            hipLaunchKernelGGL(moe_tiled_nvfp4_wide_kernel<3>, grid, dim3(TW_THREADS), 0, as_stream(stream), a);
-        else
-            hipLaunchKernelGGL(moe_tiled_nvfp4_wide_kernel<1>, grid, dim3(TW_THREADS), 0, as_stream(stream), a);
-        return launched("oom_moe_tiled_nvfp4");
-    }
-    const dim3 grid((unsigned)cdiv(n, T4_BN), (unsigned)cdiv(max_per_expert, T4_BM), (unsigned)n_experts);
-    if (precision == OOM_EXPERT_EXACT)
-        hipLaunchKernelGGL(moe_tiled_nvfp4_kernel<3>, grid, dim3(T4_THREADS), 0, as_stream(stream), a);
-    else
-        hipLaunchKernelGGL(moe_tiled_nvfp4_kernel<1>, grid, dim3(T4_THREADS), 0, as_stream(stream), a);
-    return launched("oom_moe_tiled_nvfp4");
+    const bool exact = precision == OOM_EXPERT_EXACT;
+    const TiledRoute route = tiled_route(n, k, w_off, s_off, n_experts, max_per_expert, exact);
+    const bool both = route.rows && route.tiles;
+    const TiledArgs a{recs, off, rows, x, y, n, k, w_off, s_off, s2_idx, n_experts, max_per_expert, both,
+                      tiled_grid(n, max_per_expert, route.wide),
+                      both ? tiled_cost(n, k, route.wide, exact) : TiledCost{}};
+    return exact ? launch_tiled<3>(a, route, as_stream(stream)) : launch_tiled<1>(a, route, as_stream(stream));
 }
 
 extern "C" int oom_moe_swiglu_range(const float* g, const float* u, float* h, int64_t start, int64_t end,

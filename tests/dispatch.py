@@ -32,5 +32,11 @@ def tiled(n, k, w_off, s_off, n_experts, max_n, exact):
     return ask(f"tiled {n} {k} {w_off} {s_off} {n_experts} {max_n} {int(exact)}")[0]
 
 
+def counted(n, k, wide, exact, counts, max_n=None):
+    """Which kernel the device takes where both are launched."""
+    return ask(f"counted {n} {k} {int(wide)} {int(exact)} {max_n or max(counts)} {len(counts)} "
+               + " ".join(map(str, counts)))[0]
+
+
 def step(T, E, k, hidden, inter):
     return ask(f"step {T} {E} {k} {hidden} {inter}")[0]

@@ -1,6 +1,7 @@
 // The dispatch rules of homelab_amd/csrc/dispatch.hpp as a program: one query a line on stdin,
 // one answer a line.
-//   tiled N K w_off s_off n_experts max_n exact  ->  rows | wide | narrow
+//   tiled N K w_off s_off n_experts max_n exact  ->  rows | wide | narrow | rows+wide | rows+narrow
+//   counted N K wide exact max_n n_experts n..   ->  rows | tiles (n: each expert's assignments)
 //   step T E k hidden inter                      ->  step | staged
 //   turbo kv_len kv_heads fp32                   ->  waves blocks
 #include <iostream>
@@ -16,7 +17,22 @@ int main() {
             bool exact;
             std::cin >> n >> k >> w >> s >> e >> m >> exact;
             const oom::TiledRoute r = oom::tiled_route(n, k, w, s, e, m, exact);
-            std::cout << (r == oom::TiledRoute::rows ? "rows" : r == oom::TiledRoute::wide ? "wide" : "narrow") << "\n";
+            std::cout << (r.rows ? "rows" : "") << (r.rows && r.tiles ? "+" : "")
+                      << (!r.tiles ? "" : r.wide ? "wide" : "narrow") << "\n";
+        } else if (what == "counted") {
+            int64_t n, k, m;
+            int e, t16 = 0;
+            bool wide, exact;
+            std::cin >> n >> k >> wide >> exact >> m >> e;
+            const oom::TiledGrid g = oom::tiled_grid(n, m, wide);
+            oom::XcdBlocks blocks;
+            for (int i = 0; i < e; i++) {
+                int64_t c;
+                std::cin >> c;
+                t16 += (int)oom::cdiv(c, oom::NR_M);
+                blocks.add((uint32_t)g.nx * g.ny * i, g.nx * (int32_t)oom::cdiv(c, g.rows));
+            }
+            std::cout << (oom::tiled_cost(n, k, wide, exact).rows_faster(t16, blocks) ? "rows" : "tiles") << "\n";
         } else if (what == "step") {
             int t, e, k;
             int64_t h, i;

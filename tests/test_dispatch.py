@@ -1,4 +1,5 @@
 """The host rules that pick a kernel or a split (homelab_amd/csrc/dispatch.hpp), on the CPU."""
+import numpy as np
 import pytest
 
 import dispatch
@@ -14,6 +15,63 @@ import dispatch
 ])
 def test_tiled_route(n, k, w_off, s_off, e, max_n, exact, want):
     assert dispatch.tiled(n, k, w_off, s_off, e, max_n, exact) == want
+
+
+# us a call of the few-row kernel and of the tiles it replaced, by the sizes that the host knows (n,
+# k, experts, assignments of the largest) for evenly spread picks of T tokens
+@pytest.mark.parametrize("n,k,e,max_n,exact,rows_us,tiles_us,want", [
+    (640, 2560, 64, 24, True, 40, 92, "rows"),       # 100 tokens top-10
+    (640, 2560, 128, 121, True, 185, 220, "rows"),   # 1200
+    (640, 2560, 512, 62, True, 368, 475, "rows"),    # 2048: the experts' first tiles fall on four XCDs
+    (2560, 640, 32, 33, True, 40, 28, "wide"),       # 100 top-8: one round of short tiles
+    (2560, 640, 32, 86, True, 60, 36, "wide"),       # 300
+    (2560, 640, 32, 168, False, 81, 44, "wide"),     # 600, one term
+    (1024, 512, 64, 121, False, 46, 40, "wide"),     # 600
+    (640, 2560, 64, 375, True, 295, 251, "rows+wide"),   # 2048 top-10
+    (2560, 640, 64, 375, True, 311, 252, "rows+wide"),
+    (2560, 640, 64, 682, False, 482, 328, "rows+wide"),  # 4096, one term
+    (640, 2560, 512, 108, True, 679, 594, "rows+wide"),  # 4096
+    (448, 1600, 64, 682, True, 380, 287, "rows+narrow"),
+    (1600, 448, 128, 63, True, 73, 54, "rows+narrow"),
+])
+def test_tiled_route_of_even_picks(n, k, e, max_n, exact, rows_us, tiles_us, want):
+    """The few-row kernel alone only where it is not the slower one; where both are launched the
+    device's count takes the faster one of these calls too."""
+    got = dispatch.tiled(n, k, 256, 1 << 20, e, max_n, exact)
+    assert got == want
+    assert got != "rows" or rows_us <= tiles_us
+    if "+" in got:
+        mean = int(max_n - (2 * max_n * np.log(e)) ** 0.5)
+        assert dispatch.counted(n, k, k % 128 == 0, exact, [max_n] + [mean] * (e - 1)) == "tiles"
+
+
+@pytest.mark.parametrize("n,k,exact,counts,want", [
+    # the largest expert alone does not decide: the others' few rows stay with the few-row kernel
+    (640, 2560, True, [375] + [20] * 63, "rows"),
+    (2560, 640, True, [1200] + [12] * 511, "rows"),
+    (640, 2560, False, [45] + [10] * 511, "rows"),
+    (448, 1600, True, [2000] + [9] * 63, "rows"),
+    (640, 2560, True, [320] * 64, "tiles"),
+    (640, 2560, False, [80] * 512, "tiles"),
+    (640, 2560, True, [900] * 16 + [3] * 16, "tiles"),
+    (448, 1600, True, [640] * 64, "tiles"),
+    # one tile an expert on even planes: all of them on four XCDs, two rounds where there is room for one
+    (640, 2560, True, [40, 0] * 256, "rows"),
+    (640, 2560, True, [40] * 256, "tiles"),
+])
+def test_tiled_counts(n, k, exact, counts, want):
+    assert dispatch.counted(n, k, k % 128 == 0, exact, counts, max(counts)) == want
+
+
+def test_tiled_counted_sums_are_exact():
+    """Both kernels only where every sum of the device's count is a whole number below 2^24."""
+    for e in (4, 300, 2048, 2049, 20000):
+        for max_n in (100, 5000, 200000, 3000000):
+            for n, k in ((640, 2560), (448, 1600), (20480, 2560), (65536, 320)):
+                if "+" in dispatch.tiled(n, k, 256, 1 << 20, e, max_n, True):
+                    wide = k % 128 == 0
+                    planes = -(-n // (640 if wide else 128)) * -(-max_n // (48 if wide else 64))
+                    assert e * max(-(-max_n // 16), planes) < 1 << 24 and e <= 2048
 
 
 @pytest.mark.parametrize("T,E,k,hidden,inter,want", [

@@ -10,6 +10,7 @@ same bar against the oracle's restatement. SwiGLU against numpy in f64 within 2 
 import numpy as np
 import pytest
 
+import dispatch
 import oracle
 from tiled_cases import SHAPES, case, f64_eval
 
@@ -93,26 +94,34 @@ def test_swiglu_range(hip):
     np.testing.assert_allclose(got[13:9001], want[13:9001], rtol=4e-7, atol=1e-30)
 
 
-@pytest.mark.parametrize("n,k,counts", [
-    (40, 64, [1, 16, 17]),              # one slice, fewer columns than its steps; one part of a batch
-    (130, 192, [15, 0, 33]),            # an empty expert, a second row group's first rows
-    (640, 320, [48, 2]),                # one slice filled
-    (300, 384, [16, 5]),                # two slices of 6 steps
-    (520, 1088, [7, 31]),               # four slices, the last one part filled
-    (1100, 2496, [3, 18]),              # eight slices of 10 steps, the last one part filled
-    (96, 1536, [16] * 20),              # eight slices of 6 steps, more tiles than experts' share of a block
-    (16, 128, [1, 0, 2] * 300),         # more experts than threads that count them
-    (64, 256, [200]),                   # one expert, many tiles
-    (200, 2688, [3, 50]),               # past 8 slices of 10 steps: the 48-row tiles
+@pytest.mark.parametrize("n,k,counts,route", [
+    (1024, 128, [1, 0, 2] * 200, "rows"),    # one slice, fewer columns than its 6 steps; more experts than threads
+    (1020, 192, [3, 0, 2] * 100, "rows"),    # one slice filled; rows past a row group's last subtile
+    (1030, 256, [2, 17, 0, 1] * 75, "rows"),  # one slice of 8 steps
+    (1024, 320, [5, 0, 1] * 100, "rows"),    # one slice of 10 steps
+    (300, 384, [3, 0, 16] * 100, "rows"),    # two slices of 6 steps
+    (650, 448, [5, 17, 0] * 40, "rows"),     # two slices of 8 steps, the last one part filled
+    (520, 1088, [7, 31], "rows"),            # four slices of 10, the last one part filled
+    (520, 1024, [16, 31], "rows"),           # four slices of 8, filled
+    (520, 1024, [200], "rows"),              # one expert, many tiles
+    (96, 1536, [16] * 20, "rows"),           # eight slices of 6 steps, more tiles than experts' share of a block
+    (100, 1984, [3, 18, 40], "rows"),        # eight slices of 8, the last one part filled
+    (1100, 2496, [3, 18], "rows"),           # eight slices of 10, the last one part filled
+    (640, 2560, [600], "rows"),              # one expert, many tiles and batches
+    (200, 2688, [3, 50], "wide"),            # past 8 slices of 10 steps
+    (64, 256, [120], "wide"),                # tiles filled by one expert
+    (40, 64, [1, 16, 17], "narrow"),         # short rows
+    (64, 96, [5, 60], "narrow"),             # K no whole scale words a lane
 ])
 @pytest.mark.parametrize("precision", [0, 1])
-def test_tiled_rows_kernel(hip, n, k, counts, precision):
+def test_tiled_rows_kernel(hip, n, k, counts, route, precision):
     """The few-row kernel's slices, row groups, tiles and shares at their edges (the file's f64
     bar), with the rows in any order and without a row list."""
     import torch
 
     print(f"case: tiled rows n={n} k={k} experts={len(counts)} precision={precision}", flush=True)
     recs, x, off, rows = case(n, k, counts, 5 + n + k)
+    assert dispatch.tiled(n, k, recs.w_off, recs.s_off, len(counts), max(counts), precision == 0) == route
     A = int(off[-1])
     buf = torch.from_numpy(np.stack(recs.recs)).cuda()
     addrs = torch.tensor([buf.data_ptr() + e * recs.stride for e in range(len(counts))], dtype=torch.int64,
@@ -127,3 +136,35 @@ def test_tiled_rows_kernel(hip, n, k, counts, precision):
         want, mag = f64_eval(recs, x, off, rows, precision == 0)
         assert np.isnan(got[A:]).all(), "rows past the assignments were written"
         assert (np.abs(got[:A] - want) / mag).max() < 2e-6
+
+
+@pytest.mark.parametrize("n,k,counts,bound,precision,works", [
+    (640, 2560, [1700] * 4, 1700, 0, "tiles"),          # wide tiles
+    (640, 2560, [1800] * 8, 2000, 1, "tiles"),          # a bound above the largest expert
+    (640, 2560, [1800] + [20, 0, 49] * 3, 1800, 0, "rows"),
+    (650, 2560, [17] * 40, 900, 1, "rows"),
+    (448, 1600, [1100] * 20, 1100, 0, "tiles"),         # narrow tiles
+    (448, 1600, [1100] + [7, 0, 65] * 13, 1100, 0, "rows"),
+])
+def test_tiled_counted(hip, n, k, counts, bound, precision, works):
+    """Calls that launch both kernels: whichever the count leaves working writes every row, and
+    nothing past them (the file's f64 bar)."""
+    import torch
+
+    print(f"case: tiled counted n={n} k={k} experts={len(counts)} precision={precision} {works}", flush=True)
+    recs, x, off, rows = case(n, k, counts, 11 + n + len(counts))
+    wide = k % 128 == 0
+    both = dispatch.tiled(n, k, recs.w_off, recs.s_off, len(counts), bound, precision == 0)
+    assert both == ("rows+wide" if wide else "rows+narrow")
+    assert dispatch.counted(n, k, wide, precision == 0, counts, bound) == works
+    A = int(off[-1])
+    buf = torch.from_numpy(np.stack(recs.recs)).cuda()
+    addrs = torch.tensor([buf.data_ptr() + e * recs.stride for e in range(len(counts))], dtype=torch.int64,
+                         device="cuda")
+    y = torch.full((A + 3, n), float("nan"), dtype=torch.float32, device="cuda")
+    hip.moe_tiled_nvfp4(addrs, torch.from_numpy(off).cuda(), torch.from_numpy(rows).cuda(), len(counts), bound,
+                        torch.from_numpy(x).cuda(), y, n, k, recs.w_off, recs.s_off, 0, precision)
+    got = y.cpu().numpy()
+    want, mag = f64_eval(recs, x, off, rows, precision == 0)
+    assert np.isnan(got[A:]).all(), "rows past the assignments were written"
+    assert (np.abs(got[:A] - want) / mag).max() < 2e-6
