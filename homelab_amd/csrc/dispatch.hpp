@@ -226,7 +226,9 @@ inline bool gate_up_step_ok(int T, int E, int k, int64_t hidden, int64_t inter) 
 //     the combine: 27.7 as 282 blocks of 4 waves, 18.7 as 142 of 8);
 //   - else blocks of 8 waves, at most TT_FILL in all, their waves taking more groups from there;
 //   - fp32 rows (no decoding for a second wave's MFMAs to hide behind) keep 4 waves up to two
-//     groups a wave: 17.0 us against 19.4 at 9001 keys, 2 KV heads.
+//     groups a wave (17.0 us against 19.4 at 9001 keys, 2 KV heads), and two groups a wave on
+//     blocks of 8 past that: half the blocks, and partials to combine, of one group a wave (2 KV
+//     heads, 16500 keys: 31.1 us against 35.1; 28000: 34.4 and 35.9).
 // Before, every wave was sized for two groups on blocks of 8: us a call then and now, k8v6, all
 // keys visible, 2 KV heads: 24.4 -> 15.5 at 700 keys, 24.5 -> 16.1 at 4500, 24.7 -> 18.7 at
 // 9001, 24.8 -> 19.8 at 16384, 26.2 at 32768 (the same split).
@@ -236,18 +238,19 @@ struct TurboSplit {
     int waves, blocks;
 };
 
-inline TurboSplit turbo_split(int kv_len, int kv_heads, bool fp32) {
-    const int groups = (kv_len + 15) / 16, most = std::max(1, TT_FILL / kv_heads);
-    for (int per = 4; per <= (fp32 ? 8 : 4); per += 4)
-        if ((groups + per - 1) / per <= most) return {4, (groups + per - 1) / per};
-    return {8, std::min((groups + 7) / 8, most)};
-}
-
-// Two groups a wave on blocks of 8 waves: the fewest partials, for a workspace with room for
+// Two groups a wave on blocks of 8 waves: the fewest partials, also for a workspace with room for
 // no more.
 inline TurboSplit turbo_split_least(int kv_len, int kv_heads) {
     const int groups = (kv_len + 15) / 16;
     return {8, std::max(1, std::min((groups + 15) / 16, std::max(1, TT_FILL / kv_heads)))};
+}
+
+inline TurboSplit turbo_split(int kv_len, int kv_heads, bool fp32) {
+    const int groups = (kv_len + 15) / 16, most = std::max(1, TT_FILL / kv_heads);
+    for (int per = 4; per <= (fp32 ? 8 : 4); per += 4)
+        if ((groups + per - 1) / per <= most) return {4, (groups + per - 1) / per};
+    if (fp32) return turbo_split_least(kv_len, kv_heads);
+    return {8, std::min((groups + 7) / 8, most)};
 }
 
 }  // namespace oom

@@ -113,3 +113,14 @@ def test_turbo_split_covers_the_keys():
         assert waves in (4, 8) and 1 <= blocks and (blocks == 1 or blocks * h <= 256)
         assert (blocks - 1) * waves < groups, "an empty block"
         assert waves == 8 or blocks * waves * (2 if f else 1) >= groups
+
+
+@pytest.mark.parametrize("kv_len,kv_heads,fp32,want", [
+    (8192, 2, False, "4 128"), (8193, 2, False, "8 65"), (40000, 2, False, "8 128"),
+    (8193, 2, True, "4 65"), (16384, 2, True, "4 128"),
+    # fp32 rows past two groups a wave of 4: two groups a wave of 8, half the blocks of one group
+    (16500, 2, True, "8 65"), (28000, 2, True, "8 110"), (36000, 1, True, "8 141"), (10000, 4, True, "8 40"),
+    (65536, 2, True, "8 128"),
+])
+def test_turbo_split(kv_len, kv_heads, fp32, want):
+    assert dispatch.ask(f"turbo {kv_len} {kv_heads} {int(fp32)}") == [want]
