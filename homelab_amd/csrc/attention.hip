@@ -36,8 +36,6 @@
 namespace oom {
 
 constexpr int AW = 4;           // waves per block
-constexpr int AKB = AW * 256;   // keys per block of the coarsest split
-constexpr int AG = 8;           // query heads per KV head (at most)
 constexpr int A_MAXB = 8192;    // blocks a KV head (8 Mi keys): the merge's weights sit in LDS
 constexpr int A_BUF_FLAGS = 0x00020000;
 constexpr int A_OOB = 0x7ffffff0;
@@ -441,54 +439,7 @@ __global__ void __launch_bounds__(128) attn_merge_kernel(AttnArgs a) {
 
 // ---- host side -------------------------------------------------------------------------
 
-static size_t a_al256(size_t v) { return (v + 255) & ~size_t(255); }
-
-// Splits of a KV head's keys: blocks of 4 waves with 32 NP keys a wave, NP = 1, 2, 4 or 8
-// pairs of tiles. One wave's pairs follow each other (about 1.4 us each: one pair is in
-// flight), so the finest split that still fits the chip is the fastest: at 64 / 8 heads, us a
-// step, NP = 1, 2, 4, 8 by keys
-//     1000:  8.0,  9.1, 12.1, 15.3      4096:  9.7, 10.0, 12.5, 18.7
-//     8192: 13.3, 12.1, 13.2, 18.7     16384: 17.9, 17.4, 16.6, 19.4
-//    32768: 49.1, 31.9, 30.5, 29.5     65536: 90.9, 70.9, 54.5, 54.2
-// so NP is the smallest whose blocks number at most A_FILL over all KV heads (one a CU; the
-// rows' best ends there: 4096 keys are 256 blocks at NP = 1, 8192 at NP = 2, 16384 at NP = 4)
-// and whose partials a KV head the merge takes in one round (at 1 KV head and 32768 keys, 256
-// partials: 25.3 us against 10.8 for 128 at NP = 2). Up to 256 keys one block holds the KV
-// head and no merge is launched (200 keys: 5.9 us at NP = 2 against 7.9 at NP = 1 and 13.7 at
-// NP = 8).
-constexpr int A_FILL = 256;  // blocks over all KV heads
-constexpr int A_ROUND = 128; // partials a KV head the merge loads at once
-
-struct AttnWs {
-    size_t least, total;  // what the coarsest split needs, and what every split at up to kv_len keys fits in
-};
-
-static size_t attn_part_bytes(int blocks, int kv_heads, int d) {
-    return a_al256((size_t)kv_heads * blocks * (2 * AG + AG * (size_t)d) * sizeof(float));
-}
-
-// A sequence that grows within one workspace: the finer splits of shorter sequences take at
-// most min(A_ROUND, A_FILL / kv_heads) blocks a KV head, so `total` never falls with kv_len.
-static AttnWs attn_ws(int kv_len, int kv_heads, int d) {
-    AttnWs w;
-    const int coarse = (int)cdiv(kv_len, AKB);
-    const int fine = std::min((int)cdiv(kv_len, 128), std::min(A_ROUND, A_FILL / kv_heads));
-    w.least = attn_part_bytes(coarse, kv_heads, d);
-    w.total = attn_part_bytes(std::max(coarse, fine), kv_heads, d);
-    return w;
-}
-
-// Pairs of tiles a wave (NP): the rule above, within the workspace at hand (one sized for the
-// coarsest split alone still serves).
-static int attn_pairs(int kv_len, int kv_heads, int d, size_t ws_bytes) {
-    for (int np = kv_len <= 128 ? 1 : kv_len <= 256 ? 2 : 1; np < 8; np *= 2) {
-        const int64_t blocks = cdiv(kv_len, 128 * np);
-        if (blocks == 1 || (blocks <= A_ROUND && blocks * kv_heads <= A_FILL &&
-                            attn_part_bytes((int)blocks, kv_heads, d) <= ws_bytes))
-            return np;
-    }
-    return 8;
-}
+static_assert(AKB == AW * 256, "8 pairs of tiles a wave");
 
 template <int D, int QDT, int ODT>
 static int launch_attn_t(const AttnArgs& a, int np, hipStream_t st) {
@@ -545,7 +496,7 @@ extern "C" int oom_attn_decode_paged(const void* q, int q_dtype, const uint16_t*
     a.kv_len = kv_len;
     a.Hkv = kv_heads;
     a.G = heads / kv_heads;
-    const int np = attn_pairs(kv_len, kv_heads, d, ws_bytes);
+    const int np = attn_pairs(kv_len, heads, kv_heads, d, ws_bytes);
     a.bph = (int)cdiv(kv_len, 128 * np);
     a.scale = scale;
     a.out = out;

@@ -216,6 +216,66 @@ inline bool gate_up_step_ok(int T, int E, int k, int64_t hidden, int64_t inter) 
     return items >= (per <= 1.1 ? 2.9 : hidden <= 2048 ? 4.0 : 3.5);
 }
 
+// ---- oom_attn_decode_paged (attention.hip) --------------------------------------------------
+
+constexpr int AKB = 1024;  // keys a block of the coarsest split
+constexpr int AG = 8;      // query heads per KV head (at most)
+
+// Splits of a KV head's keys: blocks of 4 waves with 32 NP keys a wave, NP = 1, 2, 4 or 8
+// pairs of tiles. One wave's pairs follow each other (about 1.4 us each: one pair is in
+// flight), so the finest split that still fits the chip is the fastest: at 64 / 8 heads, us a
+// step, NP = 1, 2, 4, 8 by keys
+//     1000:  8.0,  9.1, 12.1, 15.3      4096:  9.7, 10.0, 12.5, 18.7
+//     8192: 13.3, 12.1, 13.2, 18.7     16384: 17.9, 17.4, 16.6, 19.4
+//    32768: 49.1, 31.9, 30.5, 29.5     65536: 90.9, 70.9, 54.5, 54.2
+// so NP is the smallest whose blocks number at most A_FILL over all KV heads (one a CU; the
+// rows' best ends there: 4096 keys are 256 blocks at NP = 1, 8192 at NP = 2, 16384 at NP = 4)
+// and whose partials a KV head the merge takes in one round (at 1 KV head and 32768 keys, 256
+// partials: 25.3 us against 10.8 for 128 at NP = 2). Up to 256 keys one block holds the KV
+// head and no merge is launched (200 keys: 5.9 us at NP = 2 against 7.9 at NP = 1 and 13.7 at
+// NP = 8). The merge costs more the more query heads there are, one block a KV head does not, so
+// many of them take one block up to 1024 keys as well: NP = 4 up to 512 keys (400 keys, 8 query
+// heads a KV head, this against the finest split: 9.0 and 8.2 us at 256 query heads, 9.0 and 10.5
+// at 384, 9.6 and 18.0 at 1024), NP = 8 past that in place of two blocks (1000 keys: 15.8 and 17.4
+// at 640, 16.3 and 23.7 at 1024; with 4 a KV head 16.0 and 16.3 at 400, 16.4 and 19.5 at 512).
+constexpr int A_FILL = 256;       // blocks over all KV heads
+constexpr int A_ROUND = 128;      // partials a KV head the merge loads at once
+constexpr int A_ONE_512 = 320;    // query heads that take one block up to 512 keys,
+constexpr int A_ONE_1024 = 512;   // and in place of two up to 1024
+
+struct AttnWs {
+    size_t least, total;  // what the coarsest split needs, and what every split at up to kv_len keys fits in
+};
+
+inline size_t attn_part_bytes(int blocks, int kv_heads, int d) {
+    return ((size_t)kv_heads * blocks * (2 * AG + AG * (size_t)d) * sizeof(float) + 255) & ~size_t(255);
+}
+
+// A sequence that grows within one workspace: the finer splits of shorter sequences take at
+// most min(A_ROUND, A_FILL / kv_heads) blocks a KV head, so `total` never falls with kv_len.
+inline AttnWs attn_ws(int kv_len, int kv_heads, int d) {
+    AttnWs w;
+    const int coarse = (int)cdiv(kv_len, AKB);
+    const int fine = std::min((int)cdiv(kv_len, 128), std::min(A_ROUND, A_FILL / kv_heads));
+    w.least = attn_part_bytes(coarse, kv_heads, d);
+    w.total = attn_part_bytes(std::max(coarse, fine), kv_heads, d);
+    return w;
+}
+
+// Pairs of tiles a wave (NP): the rule above, within the workspace at hand (one sized for the
+// coarsest split alone still serves).
+inline int attn_pairs(int kv_len, int heads, int kv_heads, int d, size_t ws_bytes) {
+    if (kv_len > 256 && kv_len <= 512 && heads >= A_ONE_512) return 4;
+    for (int np = kv_len <= 128 ? 1 : kv_len <= 256 ? 2 : 1; np < 8; np *= 2) {
+        const int64_t blocks = cdiv(kv_len, 128 * np);
+        if (np == 4 && blocks == 2 && heads >= A_ONE_1024) break;
+        if (blocks == 1 || (blocks <= A_ROUND && blocks * kv_heads <= A_FILL &&
+                            attn_part_bytes((int)blocks, kv_heads, d) <= ws_bytes))
+            return np;
+    }
+    return 8;
+}
+
 // ---- oom_attn_decode_turbo (turbo.hip) ------------------------------------------------------
 
 // How a KV head's keys are dealt: blocks of `waves` waves, `blocks` of them a KV head. A wave's

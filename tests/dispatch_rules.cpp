@@ -3,6 +3,7 @@
 //   tiled N K w_off s_off n_experts max_n exact  ->  rows | wide | narrow | rows+wide | rows+narrow
 //   counted N K wide exact max_n n_experts n..   ->  rows | tiles (n: each expert's assignments)
 //   step T E k hidden inter                      ->  step | staged
+//   attn kv_len heads kv_heads ws_bytes (-1: all) ->  pairs of tiles a wave
 //   turbo kv_len kv_heads fp32                   ->  waves blocks
 #include <iostream>
 #include <string>
@@ -38,6 +39,11 @@ int main() {
             int64_t h, i;
             std::cin >> t >> e >> k >> h >> i;
             std::cout << (oom::gate_up_step_ok(t, e, k, h, i) ? "step" : "staged") << "\n";
+        } else if (what == "attn") {
+            int n, h, hk;
+            int64_t ws;
+            std::cin >> n >> h >> hk >> ws;
+            std::cout << oom::attn_pairs(n, h, hk, 128, ws < 0 ? oom::attn_ws(n, hk, 128).total : (size_t)ws) << "\n";
         } else if (what == "turbo") {
             int n, h;
             bool fp32;

@@ -124,3 +124,15 @@ def test_turbo_split_covers_the_keys():
 ])
 def test_turbo_split(kv_len, kv_heads, fp32, want):
     assert dispatch.ask(f"turbo {kv_len} {kv_heads} {int(fp32)}") == [want]
+
+
+@pytest.mark.parametrize("kv_len,heads,kv_heads,want", [
+    (100, 64, 8, 1), (200, 64, 8, 2), (700, 64, 8, 1), (4096, 64, 8, 1), (4097, 64, 8, 2), (16384, 64, 8, 4),
+    (32768, 64, 8, 8), (16384, 8, 1, 1), (16385, 8, 1, 2), (700, 32, 8, 1), (1000, 128, 128, 4),
+    # the merge of many query heads costs more than one block's longer waves
+    (257, 1024, 128, 4), (512, 1024, 128, 4), (400, 384, 48, 4), (400, 256, 32, 1), (513, 1024, 128, 8),
+    (1000, 1024, 128, 8), (1000, 640, 80, 8), (1000, 512, 128, 8), (1000, 400, 100, 4), (1000, 512, 64, 2),
+    (1025, 1024, 128, 8),
+])
+def test_attn_pairs(kv_len, heads, kv_heads, want):
+    assert dispatch.ask(f"attn {kv_len} {heads} {kv_heads} -1") == [str(want)]

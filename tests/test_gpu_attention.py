@@ -115,6 +115,7 @@ def test_attention_convex_and_page_order(hip):
     (64, 8, 4096, 16, "f32"), (64, 8, 4097, 16, "bf16"),                       # 256 blocks at NP 1; past it NP 2
     (32, 8, 8193, 32, "bf16"), (16, 8, 16385, 16, "f32"),                      # NP 4, NP 8
     (4, 1, 16385, 16, "bf16"), (4, 1, 32769, 16, "f32"),                       # past 128 partials at NP 1, at NP 2
+    (320, 40, 512, 16, "bf16"), (520, 65, 1000, 16, "f32"),                    # many heads: one block, NP 4 and NP 8
 ])
 def test_attention_split_sizes(hip, H, Hkv, kv_len, page, qdt):
     """Every split a KV head's keys can take, at the sizes where the rule changes, against f64
