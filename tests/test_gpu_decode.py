@@ -307,11 +307,12 @@ def test_fused_decode_full_size(hip, T, E, k, zipf, H, I):
     (1, 256, 32, 1040, 272, False),  # the most picks; widths ending inside a chunk
     (2, 16, 2, 16, 16, True),        # the smallest widths: most waves without an item
     (6, 64, 6, 2048, 1408, True),    # two chunks a row, mostly one token an expert
-    (5, 8, 8, 2064, 1040, True),     # four chunks, one row an item; odd groups; tiles past a chunk's end
+    (5, 8, 8, 2064, 1040, True),     # three chunks in the four-chunk kernel; odd groups; rows past a chunk's end
     (33, 8, 2, 1008, 272, False),    # bf16 past the batch kernel
-    (64, 4, 4, 4096, 144, True),     # the widest rows, every token on every expert, more down tiles than waves
+    (64, 4, 4, 4096, 144, True),     # the widest rows, every token on every expert, a down item a resident wave
     (20, 96, 8, 3072, 2048, False),  # bf16, four chunks, the widest inter
     (40, 32, 12, 512, 1024, True),   # A = 480; combine past eight slots
+    (12, 48, 8, 4096, 144, True),    # ten or more down items a wave, the last round part filled
 ])
 def test_fused_decode_general(hip, T, E, k, H, I, xf32):
     """The one-launch kernel for what the one-token and the MFMA batch kernels leave: one
@@ -337,5 +338,36 @@ def test_fused_decode_general(hip, T, E, k, H, I, xf32):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(ids.cpu().numpy(), want_ids, err_msg=f"rep {rep}")
         np.testing.assert_allclose(w.cpu().numpy(), want_w, rtol=2e-6, err_msg=f"rep {rep}")
+        err = np.abs(out.cpu().numpy() - f64).max()
+        assert err <= 2e-5 * np.abs(f64).max(), f"rep {rep}: max err {err:.3e} vs scale {np.abs(f64).max():.3e}"
+
+
+def test_fused_decode_ticket_batches(hip):
+    """256 experts of hidden 4096: 131072 down items, 64 a wave on 512 blocks of 4, so a wave takes
+    its row tiles' tickets with a full batch of lanes. Token t picks experts 32 (t % 8) .. + 31;
+    four records serve all of them. Ids as given; f32 output within 2e-5 of scale of float64."""
+    import torch
+
+    print("case: fused ticket batches T=16 E=256 k=32 H=4096 I=144", flush=True)
+    T, E, k, H, I = 16, 256, 32, 4096, 144
+    geo, hgeo = oracle.record_geometry(H, I), hip.record_geometry(H, I)
+    four = synth.expert_records(geo, 99, 4)
+    logits = np.random.default_rng(3).standard_normal((T, E)).astype(np.float32)
+    for t in range(T):
+        logits[t, 32 * (t % 8):32 * (t % 8) + 32] += 20.0
+    want_ids, want_w = oracle.router_topk(logits, k)
+    assert len(np.unique(want_ids)) == E
+    x = oracle.bf16_to_f32(synth.activations_bf16(99, T, H))
+    buf, addrs = upload_records(four)
+    addrs = addrs[torch.arange(E, device="cuda") % 4].contiguous()
+    ws = torch.zeros(hip.moe_decode_fp8_workspace_size(T, E, k, hgeo), dtype=torch.uint8, device="cuda")
+    ids = torch.empty((T, k), dtype=torch.int32, device="cuda")
+    w = torch.empty((T, k), dtype=torch.float32, device="cuda")
+    f64 = synth.f64_moe((want_ids % 4, want_w), x, four, geo)
+    for rep in range(2):
+        out = torch.full((T, H), float("nan"), dtype=torch.float32, device="cuda")
+        hip.moe_decode_fp8(dev(logits), dev(x), addrs, k, hgeo, ids, w, out, ws)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(ids.cpu().numpy(), want_ids, err_msg=f"rep {rep}")
         err = np.abs(out.cpu().numpy() - f64).max()
         assert err <= 2e-5 * np.abs(f64).max(), f"rep {rep}: max err {err:.3e} vs scale {np.abs(f64).max():.3e}"

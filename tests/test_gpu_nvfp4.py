@@ -18,6 +18,7 @@ import os
 import numpy as np
 import pytest
 
+import dispatch
 import oracle
 import synth
 
@@ -247,25 +248,32 @@ def _one_launch_check(hip, E, k, H, I, xf32, seed, logits):
     assert hip.status() == hip.OK, "a wait of the one-launch kernel gave up"
 
 
-@pytest.mark.parametrize("T,E,k,H,I,levels,xf32", [
-    (2, 64, 8, 4096, 1536, 8.0, True),     # four chunks a row; two tokens staged
-    (9, 64, 8, 4096, 768, 8.0, True),      # odd token count whose padded x overflows LDS: the staged launch
-    (8, 512, 10, 2560, 640, 8.0, False),   # three chunks
-    (13, 128, 10, 2064, 528, 2.0, True),   # odd count; rows past a whole item; widths ending inside a chunk
-    (32, 128, 16, 1008, 304, 2.0, False),  # A = 512, the plan's most, experts with many tokens
-    (33, 128, 16, 1008, 304, 2.0, False),  # A = 528: the staged launch
-    (7, 256, 4, 2048, 1552, 0.0, True),    # all logits equal: every token on the same four experts
-    (8, 300, 12, 256, 128, 2.0, False),    # routed and planned in one launch: its most tokens and slots
-    (9, 257, 3, 256, 128, 2.0, False),     # ... one token past it
-    (2, 33, 32, 256, 128, 2.0, True),      # ... A = 64; most experts chosen by both
-    (5, 64, 13, 256, 128, 2.0, True),      # ... A = 65: fewer threads a slot
+@pytest.mark.parametrize("T,E,k,H,I,levels,xf32,route", [
+    (2, 64, 8, 4096, 1536, 8.0, True, "staged"),     # four chunks a row
+    (9, 64, 8, 4096, 768, 8.0, True, "staged"),      # ... and an odd token count
+    (8, 512, 10, 2560, 640, 8.0, False, "step"),     # three chunks
+    (8, 512, 10, 2560, 640, 8.0, True, "step"),
+    (5, 512, 10, 3072, 720, 2.0, False, "step"),     # three full chunks, odd count
+    (11, 128, 10, 2064, 528, 2.0, True, "step"),     # odd count whose padded x fills LDS; width ending inside a chunk
+    (13, 128, 10, 2064, 528, 2.0, True, "staged"),   # two tokens more
+    (32, 512, 16, 1008, 304, 2.0, False, "step"),    # A = 512, the plan's most; one chunk, not filled
+    (32, 128, 16, 1008, 304, 2.0, False, "staged"),  # experts with many tokens
+    (33, 128, 16, 1008, 304, 2.0, False, "staged"),  # A = 528
+    (7, 256, 4, 2048, 1552, 0.0, True, "step"),      # all logits equal: every token on the same four experts
+    (8, 300, 12, 256, 128, 2.0, False, "staged"),    # routed and planned in one launch: its most tokens and slots
+    (9, 257, 3, 256, 128, 2.0, False, "staged"),     # ... one token past it
+    (2, 33, 32, 256, 128, 2.0, True, "staged"),      # ... A = 64; most experts chosen by both
+    (5, 64, 13, 256, 128, 2.0, True, "staged"),      # ... A = 65: fewer threads a slot
 ])
-def test_decode_nvfp4_step_matches_stages(hip, T, E, k, H, I, levels, xf32):
+def test_decode_nvfp4_step_matches_stages(hip, T, E, k, H, I, levels, xf32, route):
     """Several tokens: the step's gate/up stages all of x per block and free-runs its waves
     where x fits LDS. Its sums are the staged launch's in the staged order, so the f32 output
     equals, bit for bit, the staged launches' over the same routing. Four records serve all
-    experts (record e % 4): only the arithmetic is compared here."""
+    experts (record e % 4): only the arithmetic is compared here. `route` is what the step takes:
+    the staged rows check its routing, plan and fallback alone."""
     import torch
+
+    assert dispatch.step(T, E, k, H, I) == route
 
     print(f"case: nvfp4 step T={T} E={E} k={k} H={H} I={I} x={'f32' if xf32 else 'bf16'}", flush=True)
     seed = 1200 + T + E + H
