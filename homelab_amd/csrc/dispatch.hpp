@@ -82,44 +82,58 @@ inline TiledGrid tiled_grid(int64_t N, int64_t max_n, bool wide) {
     return {(int32_t)cdiv(N, bn), (int32_t)cdiv(max_n, bm), bm};
 }
 
-// What a projection takes by either kernel, in ns, by what its experts' assignments make of it:
-// t16 tiles of 16 for the few-row kernel, whose blocks take equal runs of the tiles' batches and load
-// a new tile's activations; rounds of one block a CU on the busiest XCD for the wide tiles; blocks
-// in flight together for the narrow ones. In whole numbers, so that every place that asks gets one
-// answer. Fitted to 4500 calls (N 256 to 4096, K 320 to 2560, 4 to 512 experts, 1 to 900 rows an
-// expert, even and skewed): half of them within 5 % of what they took, nine tenths within 20 %.
+// What a projection takes by either kernel, in ns, by what its experts' assignments make of it.
+// The few-row kernel's blocks take equal runs of its batches, t16 tiles of 16 times the batches of N:
+// a time a batch of the longest run, one a tile that the run touches (its activations load anew), one
+// a batch that the chip has in hand on average. The tiles take one a round, of one block a CU on the
+// busiest XCD (wide) or of blocks in flight together (narrow), one a block on average, and one a
+// call. In whole numbers, so that every place that asks gets one answer. Fitted to 17000 calls (N 256
+// to 4096, K 320 to 2560, 2 to 512 experts, 1 to 900 rows an expert, even and skewed): nine tenths of
+// the few-row kernel's are within 11 % of what they took, of the wide tiles' within 18 %.
 struct TiledCost {
-    int32_t start, batch, tile, batches;  // few-row kernel
-    int32_t once, round;                  // tiles
+    int32_t start, batch, tile, flow, batches;  // few-row kernel
+    int32_t once, round, block;                 // tiles
     bool wide;
     OOM_HD int64_t rows_ns(int32_t t16) const {
-        return start + batch * (((int64_t)t16 * batches + 255) >> 8) + ((int64_t)tile * t16 >> 8);
+        const int64_t all = (int64_t)t16 * batches;
+        const int32_t run = all > 256 ? (int32_t)((all + 255) >> 8) : 1;
+        return start + (int64_t)batch * run + (int64_t)tile * (1 + (run + batches - 2) / batches) + (flow * all >> 8);
     }
     OOM_HD int64_t tiles_ns(const XcdBlocks& blocks) const {
         int32_t most = 0;
-        for (int i = 0; i < 8; i++) most = blocks.on[i] > most ? blocks.on[i] : most;
-        return once + (wide ? (int64_t)round * ((most + 31) >> 5) : (int64_t)round * (most > 32 ? most : 32) >> 5);
+        int64_t all = 0;
+        for (int i = 0; i < 8; i++) {
+            all += blocks.on[i];
+            most = blocks.on[i] > most ? blocks.on[i] : most;
+        }
+        const int64_t rounds = wide ? (most + 31) / 32 * 32 : most > 32 ? most : 32;
+        return once + (round * rounds >> 5) + (block * all >> 8);
     }
-    OOM_HD bool rows_faster(int32_t t16, const XcdBlocks& blocks) const { return rows_ns(t16) <= tiles_ns(blocks); }
+    // (a twentieth of difference goes to the few-row kernel: skewed picks are the worse to get wrong)
+    OOM_HD bool rows_faster(int32_t t16, const XcdBlocks& blocks) const {
+        return 20 * rows_ns(t16) <= 21 * tiles_ns(blocks);
+    }
 };
 inline TiledCost tiled_cost(int64_t N, int64_t K, bool wide, bool exact) {
     const RowsSplit sp = rows_split(K);
-    TiledCost c;
-    c.batches = rows_batches(N, sp);
-    const int i = sp.st == 6 ? 0 : sp.st == 8 ? 1 : 2;
-    const int32_t rows[2][3][3] = {{{5600, 5560, 3800}, {6400, 6860, 4800}, {6900, 8900, 5600}},
-                                   {{5600, 6880, 3800}, {6600, 8340, 5000}, {9600, 11000, 6300}}};
-    c.start = rows[exact][i][0], c.batch = rows[exact][i][1], c.tile = rows[exact][i][2];
+    const int32_t rows[2][3][4] = {{{4099, 2176, 4154, 3143}, {4423, 2311, 5144, 4224}, {4820, 3100, 6205, 5329}},
+                                   {{4213, 3205, 4274, 3379}, {4704, 3626, 5173, 4437}, {6674, 4960, 7362, 5524}}};
+    const int32_t* const r = rows[exact][sp.st == 6 ? 0 : sp.st == 8 ? 1 : 2];
     const int32_t k = (int32_t)K;
-    if (wide) {  // waves past N are idle: of the round's time per column, a part goes with the rows there are
-        const int32_t full = (int32_t)(k * N / (TW_BN * cdiv(N, TW_BN)));
-        c.once = exact ? -75 * k / 10 : -69 * k / 10;
-        c.round = exact ? 5050 + (345 * k + 87 * full) / 10 : 3900 + (202 * k + 122 * full) / 10;
-    } else {
-        c.once = exact ? 68 * k / 10 : 29 * k / 10;
-        c.round = exact ? 190 + 162 * k / 10 : 146 * k / 10 - 390;
-    }
+    TiledCost c;
+    c.start = r[0], c.batch = r[1], c.tile = r[2], c.flow = r[3];
+    c.batches = rows_batches(N, sp);
     c.wide = wide;
+    if (wide) {  // waves past N are idle: a part of a round goes with the rows there are
+        const int32_t full = (int32_t)(k * N / (TW_BN * cdiv(N, TW_BN)));
+        c.once = exact ? -228 * k / 100 : -126 * k / 100;
+        c.round = exact ? 4825 + (2836 * k + 777 * full) / 100 : 3613 + (1348 * k + 1137 * full) / 100;
+        c.block = exact ? 753 * k / 100 : 817 * k / 100;
+    } else {
+        c.once = exact ? 984 * k / 100 : 567 * k / 100;
+        c.round = exact ? 557 + 1105 * k / 100 : std::max(0, 899 * k / 100 - 672);
+        c.block = exact ? 452 * k / 100 : 592 * k / 100;
+    }
     return c;
 }
 
@@ -137,9 +151,10 @@ struct TiledRoute {
 // first tiles alone can fall on half of the XCDs. So: the few-row kernel where it is the faster one
 // of evenly spread picks, the tiles where they are with every expert but one in a single tile, both
 // between the two. The second launch and the counting cost 3.3 us and 1 us a round of tiles, so a
-// call whose tiles take less than TR_COUNT_NS takes one kernel alone, as does one whose evenly spread
-// picks make a twentieth of difference, one with more experts than a block counts in a few loads, or
-// one with sums past 2^24 (the device's are f32).
+// call whose tiles take less than TR_COUNT_NS takes them alone, as does one with more experts than a
+// block counts in a few loads, or with sums past 2^24 (the device's are f32). On average over the
+// calls above this takes 1.02 of the faster kernel's time for evenly spread picks and 1.03 to 1.05
+// for skewed ones; the few-row kernel wherever N and K fill its slices took 1.06 and 1.06 to 1.09.
 constexpr int64_t TR_COUNT_NS = 50000;
 constexpr int TR_COUNT_E = 2048;
 inline TiledRoute tiled_route(int64_t N, int64_t K, int64_t w_off, int64_t s_off, int64_t n_experts, int64_t max_n,
@@ -168,12 +183,11 @@ inline TiledRoute tiled_route(int64_t N, int64_t K, int64_t w_off, int64_t s_off
     };
     const int64_t t16 = tiles(NR_M), tn = tiles(grid.rows);
     const XcdBlocks even = blocks(tn / n_experts, tn % n_experts);
-    const int64_t ns = cost.tiles_ns(even);
-    if (cost.rows_ns((int32_t)t16) <= ns + (ns < TR_COUNT_NS ? 0 : ns / 20)) return {true, false, wide};
+    if (cost.rows_faster((int32_t)t16, even)) return {true, false, wide};
     XcdBlocks skewed = blocks(1, 0);
     skewed.add(0, grid.nx * (grid.ny - 1));
     const int64_t sums = n_experts * std::max(cdiv(max_n, NR_M), (int64_t)grid.nx * grid.ny);
-    if (n_experts > TR_COUNT_E || sums >= 1 << 24 || ns < TR_COUNT_NS ||
+    if (n_experts > TR_COUNT_E || sums >= 1 << 24 || cost.tiles_ns(even) < TR_COUNT_NS ||
         !cost.rows_faster((int32_t)(cdiv(max_n, NR_M) + n_experts - 1), skewed))
         return {false, true, wide};
     return {true, true, wide};
@@ -282,8 +296,9 @@ inline int attn_pairs(int kv_len, int heads, int kv_heads, int d, size_t ws_byte
 // groups follow each other (about 4 us each: 128 fp32 MFMAs and the decoding between them), so
 // every wave takes one group as long as the grid then has a block a CU or fewer:
 //   - blocks of 4 waves, one a SIMD, while ceil(groups / 4) blocks a KV head make at most
-//     TT_FILL in all; past that two of them share a CU (9001 keys, 2 KV heads, us a call with
-//     the combine: 27.7 as 282 blocks of 4 waves, 18.7 as 142 of 8);
+//     TT_FILL in all; past that some CUs have a second round of them (a wave's 340 registers leave
+//     a SIMD no room for another; 9001 keys, 2 KV heads, us a call with the combine: 27.7 as 282
+//     blocks of 4 waves, 18.7 as 142 of 8);
 //   - else blocks of 8 waves, at most TT_FILL in all, their waves taking more groups from there;
 //   - fp32 rows (no decoding for a second wave's MFMAs to hide behind) keep 4 waves up to two
 //     groups a wave (17.0 us against 19.4 at 9001 keys, 2 KV heads), and two groups a wave on

@@ -23,6 +23,7 @@ def test_tiled_route(n, k, w_off, s_off, e, max_n, exact, want):
     (640, 2560, 64, 24, True, 40, 92, "rows"),       # 100 tokens top-10
     (640, 2560, 128, 121, True, 185, 220, "rows"),   # 1200
     (640, 2560, 512, 62, True, 368, 475, "rows"),    # 2048: the experts' first tiles fall on four XCDs
+    (704, 1152, 128, 13, False, 22, 30, "rows"),     # 68, one term: a round of tiles on every CU
     (2560, 640, 32, 33, True, 40, 28, "wide"),       # 100 top-8: one round of short tiles
     (2560, 640, 32, 86, True, 60, 36, "wide"),       # 300
     (2560, 640, 32, 168, False, 81, 44, "wide"),     # 600, one term
