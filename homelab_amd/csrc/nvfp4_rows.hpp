@@ -7,7 +7,7 @@
 // loop and no wave waits for another there. (Activations staged through LDS per K block, with
 // the weights' loads in the operand layout or transposed through LDS, took 225-245 us for 512
 // experts of 640 x 2560 with 10 rows each, whatever the occupancy: the loop was a chain of LDS
-// reads, decoding and barriers. This form takes 147.)
+// reads, decoding and barriers. This form takes 147 to 158.)
 //
 //   - slice s of KS takes K columns [32 ST s, 32 ST (s + 1)); lane (r, q) (r = lane % 16, q =
 //     lane / 16) holds the 8 ST columns from 32 ST s + 8 ST q on, of activation row r and of
@@ -32,7 +32,8 @@ typedef __bf16 n4bf16x2 __attribute__((ext_vector_type(2)));
 typedef float n4f32x2 __attribute__((ext_vector_type(2)));
 typedef float n4f4 __attribute__((ext_vector_type(4)));
 
-// Two f32 values as packed bf16 (round to nearest even).
+// Two f32 values as packed bf16 (v_cvt_pk_bf16_f32, round to nearest even; exact for the weights
+// here, which are bf16 values).
 __device__ __forceinline__ uint32_t n4_cvt(float lo, float hi) {
     const n4f32x2 v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, n4bf16x2));

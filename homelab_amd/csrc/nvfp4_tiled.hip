@@ -80,16 +80,6 @@ __device__ __forceinline__ bool counted_rows_faster(const TiledArgs& g) {
     return g.cost.rows_faster(total(8), blocks);
 }
 
-typedef __bf16 t4bf16x2 __attribute__((ext_vector_type(2)));
-typedef float t4f32x2 __attribute__((ext_vector_type(2)));
-
-// Two f32 values as packed bf16 (v_cvt_pk_bf16_f32, round to nearest even; exact for the
-// weights here, which are bf16 values).
-__device__ __forceinline__ uint32_t t4_cvt(float lo, float hi) {
-    const t4f32x2 v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, t4bf16x2));
-}
-
 template <int TERMS>
 __global__ void __launch_bounds__(T4_THREADS, 2) moe_tiled_nvfp4_kernel(TiledArgs g) {
     __shared__ __align__(16) uint16_t wsh[2][T4_BN][T4_LS];
@@ -153,10 +143,10 @@ __global__ void __launch_bounds__(T4_THREADS, 2) moe_tiled_nvfp4_kernel(TiledArg
             const auto p1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw[i], 1.0f, 1);
             const auto p2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw[i], 1.0f, 2);
             const auto p3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw[i], 1.0f, 3);
-            packed[4 * i] = t4_cvt(p0[0] * sc, p0[1] * sc);
-            packed[4 * i + 1] = t4_cvt(p1[0] * sc, p1[1] * sc);
-            packed[4 * i + 2] = t4_cvt(p2[0] * sc, p2[1] * sc);
-            packed[4 * i + 3] = t4_cvt(p3[0] * sc, p3[1] * sc);
+            packed[4 * i] = n4_cvt(p0[0] * sc, p0[1] * sc);
+            packed[4 * i + 1] = n4_cvt(p1[0] * sc, p1[1] * sc);
+            packed[4 * i + 2] = n4_cvt(p2[0] * sc, p2[1] * sc);
+            packed[4 * i + 3] = n4_cvt(p3[0] * sc, p3[1] * sc);
         }
         uint4* dst = reinterpret_cast<uint4*>(&wsh[b][wr][16 * wh]);
         dst[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
@@ -170,7 +160,7 @@ __global__ void __launch_bounds__(T4_THREADS, 2) moe_tiled_nvfp4_kernel(TiledArg
             float v[4] = {x4.x, x4.y, x4.z, x4.w};
 #pragma unroll
             for (int p = 0; p < TERMS; p++) {
-                const uint32_t w0 = t4_cvt(v[0], v[1]), w1 = t4_cvt(v[2], v[3]);
+                const uint32_t w0 = n4_cvt(v[0], v[1]), w1 = n4_cvt(v[2], v[3]);
                 *reinterpret_cast<uint2*>(&xsh[b][p][t][kq]) = make_uint2(w0, w1);
                 if (p + 1 < TERMS) {
                     v[0] -= __uint_as_float(w0 << 16);
@@ -332,7 +322,7 @@ __global__ void __launch_bounds__(TW_THREADS) moe_tiled_nvfp4_wide_kernel(TiledA
             float v[4] = {x4.x, x4.y, x4.z, x4.w};
 #pragma unroll
             for (int p = 0; p < TERMS; p++) {
-                const uint32_t w0 = t4_cvt(v[0], v[1]), w1 = t4_cvt(v[2], v[3]);
+                const uint32_t w0 = n4_cvt(v[0], v[1]), w1 = n4_cvt(v[2], v[3]);
                 *reinterpret_cast<uint2*>(&xsh[b][p][m][kq]) = make_uint2(w0, w1);
                 if (p + 1 < TERMS) {
                     v[0] -= __uint_as_float(w0 << 16);
@@ -362,8 +352,8 @@ __global__ void __launch_bounds__(TW_THREADS) moe_tiled_nvfp4_wide_kernel(TiledA
                 const auto p2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw, 1.0f, 2);
                 const auto p3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(cw, 1.0f, 3);
                 bop[ns] = __builtin_bit_cast(
-                    t4bf16x8, make_uint4(t4_cvt(p0[0] * sc, p0[1] * sc), t4_cvt(p1[0] * sc, p1[1] * sc),
-                                         t4_cvt(p2[0] * sc, p2[1] * sc), t4_cvt(p3[0] * sc, p3[1] * sc)));
+                    t4bf16x8, make_uint4(n4_cvt(p0[0] * sc, p0[1] * sc), n4_cvt(p1[0] * sc, p1[1] * sc),
+                                         n4_cvt(p2[0] * sc, p2[1] * sc), n4_cvt(p3[0] * sc, p3[1] * sc)));
             }
 #pragma unroll
             for (int ms = 0; ms < TW_MS; ms++) {
@@ -422,9 +412,10 @@ __global__ void __launch_bounds__(TW_THREADS) moe_tiled_nvfp4_wide_kernel(TiledA
 // (nvfp4_rows.hpp) One block a CU. The blocks count every expert's 16-row tiles, times the
 // batches of 128 weight rows a row group that a projection has, and each takes an equal run of
 // those units, so no CU waits for a last round of blocks: 511 experts' tiles and 14 second
-// ones as a block each took 180 us a projection of 640 x 2560, the equal runs 147. What bounds
+// ones as a block each took 180 us a projection of 640 x 2560, the equal runs 147 to 158. What bounds
 // it there: the decoding and the matrix cores of two waves a SIMD (184 vector instructions and
-// 30 MFMAs a 16-row subtile and slice, about 90 us) beside the stream (77 us at 6.1 TB/s).
+// 30 MFMAs a 16-row subtile and slice, about 90 us) beside the stream (77 us at 6.1 TB/s). With ten
+// steps and three terms 42 registers spill, outside the subtiles' loop: a tile reloads them once.
 constexpr int TR_LIST = 1024;  // tiles a block can have
 
 template <int TERMS, int ST>

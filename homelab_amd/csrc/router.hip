@@ -429,15 +429,15 @@ int launch_plan_multi(const int32_t* ids, int T, int E, int k, const uint64_t* a
 //
 // Both are chains of short latencies (6.4 us and 8 us as two launches at 8 tokens, 512
 // experts, top-10), so one block does both: a wave routes a token (route_token_regs), and
-// with the ids in LDS every slot's place comes from comparisons with all slots, P = 1024 /
-// (slots rounded up to a power of two) threads a slot: no counts, scans or rounds. NVFP4
-// decode step: 40.0 -> 35.1 us at 2 tokens of that, 87.9 -> 85 at 8, 20.0 -> 15.6 at 2 tokens
+// with the ids in LDS every slot's place comes from comparisons with all slots, P threads a
+// slot (16 up to 64 slots, 8 past that): no counts, scans or rounds. NVFP4
+// decode step: 40.0 -> 35.1 us at 2 tokens of that, 87.9 -> 83.2 at 8, 20.0 -> 15.6 at 2 tokens
 // of 64 experts top-4, 1024 / 256.
 // The line: past two tokens a SIMD the one CU routes slower than a block a token does (16
 // tokens of 256 experts top-6, 1024 / 256: 38.2 against 37.4 us; of 512 top-10: 167 and 163).
 constexpr int RP_T = 8;      // a wave a token
 constexpr int RP_A = 96;     // slots
-constexpr int RP_LDS = 128;  // slots rounded up to 4 P
+constexpr int RP_LDS = 128;  // slots in whole reads of 4 by P threads
 template <int EQ>
 __global__ void __launch_bounds__(1024) route_plan_kernel(const float* __restrict__ logits, int T, int E, int k,
                                                           const uint64_t* __restrict__ all_recs,

@@ -658,7 +658,7 @@ __global__ void __launch_bounds__(TW * 64) attn_turbo_kernel(TurboArgs a) {
     const __amdgpu_buffer_rsrc_t qr = tq_rsrc(a.q + (size_t)kvh * G * D, G * D * 4);
     const uint32_t b0 = tq_mask_byte(mr, a.kv_len, ngroups, wv, W, 0, lane);
     const uint32_t b1 = tq_mask_byte(mr, a.kv_len, ngroups, wv, W, 1, lane);
-    // wave w rotates heads w and w + 8 (rows 12 .. 15 are zero); lane l holds coordinates
+    // wave w rotates heads w, w + TW, ... (rows 12 .. 15 are zero); lane l holds coordinates
     // 4 l .. 4 l + 3
     constexpr int NJ = 16 / TW;
     uint4 qh[NJ];

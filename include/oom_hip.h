@@ -338,7 +338,10 @@ int oom_moe_swiglu_range(const float* g, const float* u, float* h, int64_t start
  * j % page_size. d = 128, heads / kv_heads <= 8, page_size a multiple of 16. fp32 dot
  * products, exp and accumulation (fp32 q enters the bf16 matrix cores as an exact
  * three-term split); out [heads, d] in out_dtype. Every key up to kv_len is visible
- * (the decode position is the last one).
+ * (the decode position is the last one). How the keys are split, and so the order of the
+ * sums, follows from the sizes and ws_bytes: a workspace below the size given is accepted
+ * down to that of the coarsest split, one block a KV head and 1024 keys, and splits so far
+ * as it has room.
  * Replaces Attention::attention at decode (crates/oominf-core/src/backend.rs:545-568;
  * crates/oominf-cuda/src/attention.rs:265-346, which routes D=128, G=8 to attn_prefill,
  * crates/oominf-cuda/kernels/attention.cu:419-553), over a paged bf16 cache. */
@@ -383,7 +386,9 @@ int oom_mask_compact(const uint8_t* mask, int32_t* sel, int n, void* stream);
  * 256] (rotated on the device for a Turbo cache), the keys j < kv_len with mask[j] != 0
  * (u8 [kv_len]), out f32 [heads, 256] = sum_j softmax_j(q_h . k_j * scale) v_j (rotated
  * back), query head h reading KV head h / 12. k_bits and v_bits both 0 or both 2..8.
- * fp32 dot products, exp and accumulation. */
+ * fp32 dot products, exp and accumulation. The keys' split follows from the sizes and
+ * ws_bytes, as in oom_attn_decode_paged: below the size given, a workspace with room for
+ * blocks of 256 keys (at most 256 over the KV heads) is accepted and gets those. */
 size_t oom_attn_decode_turbo_workspace_size(int heads, int kv_heads, int d, int kv_len);
 int oom_attn_decode_turbo(const float* q, const uint8_t* k, const uint8_t* v, int k_bits, int v_bits,
                           const float* levels, const uint8_t* mask, int heads, int kv_heads, int d, int kv_len,
