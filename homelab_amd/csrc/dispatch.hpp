@@ -214,6 +214,10 @@ constexpr int64_t N4S_XMAX = 144 * 1024; // of LDS for the tokens' x, beside the
 //     47.8, 46.0; 6.3, 1.9: 84.2, 78.5; 10.3, 1.6: 118, 103
 //   one (1024 / 512), where the decoding weighs most: 2.0, 6.0: 57.3, 61.5; 4.0, 4.1: 67.6, 72.2;
 //     5.2, 1.6: 50.9, 50.9; 7.0, 2.3: 69.9, 74.0; 8.7, 1.2: 70.1, 66.6; 15, 1.3: 115, 108
+// Skewed picks reach fewer experts, so the lines lie above where even ones break even: over 420
+// random steps (215 of even picks, 110 and 95 of popularity falling with rank to the 0.5 and 1.1) this
+// takes 0.989, 0.997 and 1.000 of the staged time; lines at the break-even 0.990, 1.001 and 1.002, with
+// 34 steps more than 2 % slower in place of 11.
 constexpr int64_t N4S_MAX_H = 3072;
 constexpr int N4S_WAVES = 8;    // waves a block, on one block a CU
 constexpr int N4S_GRID = 256;
@@ -226,8 +230,8 @@ inline bool gate_up_step_ok(int T, int E, int k, int64_t hidden, int64_t inter) 
     if (A > N4S_AMAX || hidden > N4S_MAX_H || gate_up_step_lds(T, hidden) > N4S_XMAX) return false;
     const double experts = E * (1.0 - std::pow(1.0 - (double)k / E, T));
     const double items = experts * (double)cdiv(inter, N4S_ROWS) / (N4S_GRID * N4S_WAVES), per = A / experts;
-    if (hidden <= 1024) return items >= (per <= 1.75 ? 5.0 : 8.0);
-    return items >= (per <= 1.1 ? 2.9 : hidden <= 2048 ? 4.0 : 3.5);
+    if (hidden <= 1024) return items >= (per <= 1.15 ? 7.0 : 10.0);
+    return items >= (hidden <= 2048 ? 5.0 : per <= 1.1 ? 2.9 : 4.0);
 }
 
 // ---- oom_attn_decode_paged (attention.hip) --------------------------------------------------

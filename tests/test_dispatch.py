@@ -95,6 +95,11 @@ def test_tiled_counted_sums_are_exact():
     (32, 512, 10, 1024, 512, "step"),
     (16, 128, 8, 2048, 1536, "step"),
     (16, 64, 8, 2048, 1536, "step"),
+    # near the break-even of even picks, where skewed ones lose
+    (17, 256, 8, 1168, 336, "staged"),
+    (18, 64, 8, 1184, 656, "staged"),
+    (19, 256, 8, 880, 464, "staged"),
+    (9, 128, 8, 2240, 544, "staged"),
     # past the plan's 512 slots; x past its LDS
     (33, 128, 16, 1008, 304, "staged"),
     (13, 512, 10, 2560, 640, "staged"),
