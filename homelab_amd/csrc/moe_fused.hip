@@ -103,8 +103,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rec_rsrc(const PlanLds& pl, in
 // wave's next item (gate/up or down) loads behind the current one's sums; an expert's first
 // token (the only one of most, at a few tokens) takes a pass of its own, its activations
 // loaded in one round ahead of the next item's rows, and the others go two a pass (four: 161
-// against 151 us at 16 tokens of the case below, and spills with f32 rows of 4096). All of a
-// wave's tickets are taken together after its last down item. Before, an item's loads went
+// against 151 us at 16 tokens of the case below, and spills with f32 rows of 4096), or four
+// where a chunk of 1024 columns holds a row of either width and the registers hold four (16
+// experts top-4, 1024 / 512, 4 tokens: 27.9 us two a pass, 25.2; top-8, 20 tokens: 71.8 and
+// 67.2). All of a wave's tickets are taken together after its last down item. Before, an item's loads went
 // out one item at a time through flat addresses, every pass did four tokens' sums in down,
 // and a ticket's round trip followed each item. 64 experts top-6, 2048 / 1408, f32: 97 -> 79
 // us at 6 tokens (240 MB, 37 us at the stream's rate), 173 -> 150 at 16, 305 -> 271 at 40;
@@ -231,7 +233,7 @@ __device__ __forceinline__ void gate_up_put(const FusedArgs& a, int a0, int nb, 
 // The whole of phase 1 for one wave.
 template <int XDT, int CS>
 __device__ __forceinline__ void gate_up_phase(const FusedArgs& a, const PlanLds& pl, int n_e, int gwave, int NW, int lane) {
-    constexpr int R = FG_R, TG = 2, ES = XDT == OOM_BF16 ? 2 : 4;
+    constexpr int R = FG_R, TG = CS == 1 ? 4 : 2, ES = XDT == OOM_BF16 ? 2 : 4;
     const int H = (int)a.H;
     const int tiles_g = (int)((a.I + R - 1) / R), NG = n_e * tiles_g;
     const __amdgpu_buffer_rsrc_t xr =
@@ -282,22 +284,24 @@ __device__ __forceinline__ void gate_up_phase(const FusedArgs& a, const PlanLds&
     }
 }
 
-// The weights and scales of down item `it` (expert it / tiles_d): 8 rows x 2 chunks of 1024
+// The weights and scales of down item `it` (expert it / tiles_d): 8 rows x DC chunks of 1024
 // columns per lane; an item past ND reads zeros.
+template <int DC>
 struct DownW {
-    uint4 w[FD_R][2];
-    float s[2];
+    uint4 w[FD_R][DC];
+    float s[DC];
 };
 
+template <int DC>
 __device__ __forceinline__ void down_load(const FusedArgs& a, const PlanLds& pl, int it, int ND, int tiles_d, int lane,
-                                          DownW& d) {
+                                          DownW<DC>& d) {
     const int H = (int)a.H, I = (int)a.I, nkb = (I + 127) >> 7;
     const bool valid = it < ND;
     const int i = __builtin_amdgcn_readfirstlane(valid ? it / tiles_d : 0);
     const int r0 = __builtin_amdgcn_readfirstlane(valid ? (it - i * tiles_d) * FD_R : 0);
     const __amdgpu_buffer_rsrc_t r = rec_rsrc(pl, i, valid ? a.rec_bytes : 0);
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
+    for (int c = 0; c < DC; c++) {
         const int col = c * 1024 + lane * 16;
         const bool ok = valid && col < I;
 #pragma unroll
@@ -309,14 +313,14 @@ __device__ __forceinline__ void down_load(const FusedArgs& a, const PlanLds& pl,
 
 // h of assignments a0 .. a0 + nb (zeros past nb) for this lane's 2 chunks of 16
 // columns, through device-coherent 128-bit buffer loads.
-template <int TG>
-__device__ __forceinline__ void down_h_load(const FusedArgs& a, int a0, int nb, int lane, float (&hv)[TG][2][16]) {
+template <int TG, int DC>
+__device__ __forceinline__ void down_h_load(const FusedArgs& a, int a0, int nb, int lane, float (&hv)[TG][DC][16]) {
     const int I = (int)a.I;
     const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(a.h, (short)0, a.h_bytes, BUF_FLAGS);
 #pragma unroll
     for (int t = 0; t < TG; t++)
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
+        for (int c = 0; c < DC; c++) {
             const int col = c * 1024 + lane * 16;
             const int off = t < nb && col < I ? ((a0 + t) * I + col) * 4 : OOB;
 #pragma unroll
@@ -331,13 +335,13 @@ __device__ __forceinline__ void down_h_load(const FusedArgs& a, int a0, int nb, 
 }
 
 // y[a0 + t, r0 .. r0 + FD_R) = h . Wd rows for the token group, from loaded weights and h.
-template <int TG>
-__device__ __forceinline__ void down_rows(const FusedArgs& a, int r0, int lane, const DownW& d,
-                                          const float (&hv)[TG][2][16], int a0, int nb) {
+template <int TG, int DC>
+__device__ __forceinline__ void down_rows(const FusedArgs& a, int r0, int lane, const DownW<DC>& d,
+                                          const float (&hv)[TG][DC][16], int a0, int nb) {
     const int H = (int)a.H;
     float acc[TG * FD_R] = {};
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
+    for (int c = 0; c < DC; c++) {
         if (c * 1024 >= (int)a.I) break;
 #pragma unroll
         for (int r = 0; r < FD_R; r++) {
@@ -387,23 +391,24 @@ __device__ __forceinline__ void combine_tile(const FusedArgs& a, const PlanLds& 
 // Phase 2 for one wave, its first item's weights already loading in wa: the y rows of its
 // items, then the tickets of their row tiles (a lane each, 64 items at a time) once the
 // wave's y stores completed; the taker of a tile's last ticket combines it.
-template <int ODT>
+template <int ODT, int DC>
 __device__ __forceinline__ void down_phase(const FusedArgs& a, const PlanLds& pl, int n_e, int ND, int tiles_d, int gwave,
-                                           int NW, int lane, DownW& wa) {
-    const auto item = [&](int it, const DownW& d, DownW& next) {
+                                           int NW, int lane, DownW<DC>& wa) {
+    const auto item = [&](int it, const DownW<DC>& d, DownW<DC>& next) {
         const int i = __builtin_amdgcn_readfirstlane(it / tiles_d), r0 = (it - i * tiles_d) * FD_R;
         const int a0 = __builtin_amdgcn_readfirstlane(pl.off[i]), a1 = __builtin_amdgcn_readfirstlane(pl.off[i + 1]);
         {
-            float hv[1][2][16];
-            down_h_load<1>(a, a0, 1, lane, hv);
-            down_load(a, pl, it + NW, ND, tiles_d, lane, next);
-            down_rows<1>(a, r0, lane, d, hv, a0, 1);
+            float hv[1][DC][16];
+            down_h_load<1, DC>(a, a0, 1, lane, hv);
+            down_load<DC>(a, pl, it + NW, ND, tiles_d, lane, next);
+            down_rows<1, DC>(a, r0, lane, d, hv, a0, 1);
         }
-        for (int as = a0 + 1; as < a1; as += 2) {
-            const int nb = min(2, a1 - as);
-            float hv[2][2][16];
-            down_h_load<2>(a, as, nb, lane, hv);
-            down_rows<2>(a, r0, lane, d, hv, as, nb);
+        constexpr int TG = DC == 1 ? 4 : 2;
+        for (int as = a0 + 1; as < a1; as += TG) {
+            const int nb = min(TG, a1 - as);
+            float hv[TG][DC][16];
+            down_h_load<TG, DC>(a, as, nb, lane, hv);
+            down_rows<TG, DC>(a, r0, lane, d, hv, as, nb);
         }
     };
     const auto flush = [&](int first, int n) {  // the tickets of items first, first + NW, ... (n <= 64)
@@ -419,7 +424,7 @@ __device__ __forceinline__ void down_phase(const FusedArgs& a, const PlanLds& pl
             combine_tile<ODT>(a, pl, __builtin_amdgcn_readlane(tile, l), lane);
         }
     };
-    DownW wb;
+    DownW<DC> wb;
     int first = gwave, n = 0;
     for (int it = gwave; it < ND; it += 2 * NW) {
         item(it, wa, wb);
@@ -923,11 +928,12 @@ __global__ void __launch_bounds__(TG == 1 ? 64 * FW1 : 64 * FW, 2) moe_decode_fu
         gate_up_phase<XDT, DCH>(a, pl, n_e, gwave, NW, lane);
         wait_mem();  // this wave's h stores are complete before its block arrives
         // ---- the first down item's weights stream while the grid meets ----
-        DownW d;
-        down_load(a, pl, gwave, ND, tiles_d, lane, d);
+        constexpr int DC = DCH == 1 ? 1 : 2;
+        DownW<DC> d;
+        down_load<DC>(a, pl, gwave, ND, tiles_d, lane, d);
         grid_barrier(a, bbase);
         // ---- phase 2: down projection -> y, then the ticketed slot-order combine ----
-        down_phase<ODT>(a, pl, n_e, ND, tiles_d, gwave, NW, lane, d);
+        down_phase<ODT, DC>(a, pl, n_e, ND, tiles_d, gwave, NW, lane, d);
     }
     grid_barrier_exit(a.bar);
 }
@@ -1041,7 +1047,8 @@ int launch_fused(const float* logits, const void* x, int xdt, const uint64_t* al
     if (xdt == OOM_F32 && odt == OOM_BF16) return launch_fused_t<TG, DCH, EQ, OOM_F32, OOM_BF16>(a, lds, st);   \
     return launch_fused_t<TG, DCH, EQ, OOM_F32, OOM_F32>(a, lds, st);
     // one token routed to at most FW1 experts: TG 1 with 512-column down chunks for the
-    // inter width; otherwise TG 4 with 1024-column chunks for the hidden width
+    // inter width; otherwise TG 4 with 1024-column chunks for the hidden width, and one for
+    // the inter width where both are one
     if (T == 1 && k <= FW1) {
         if (E <= 128) {
             if (g.inter <= 1024) {
@@ -1060,6 +1067,8 @@ int launch_fused(const float* logits, const void* x, int xdt, const uint64_t* al
                 FUSED_CASE(1, 4, 4)
             }
         }
+    } else if (g.hidden <= 1024 && g.inter <= 1024) {
+        FUSED_CASE(4, 1, 4)
     } else if (g.hidden <= 2048) {
         FUSED_CASE(4, 2, 4)
     } else {

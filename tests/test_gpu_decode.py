@@ -309,6 +309,9 @@ def test_fused_decode_full_size(hip, T, E, k, zipf, H, I):
     (6, 64, 6, 2048, 1408, True),    # two chunks a row, mostly one token an expert
     (5, 8, 8, 2064, 1040, True),     # three chunks in the four-chunk kernel; odd groups; rows past a chunk's end
     (33, 8, 2, 1008, 272, False),    # bf16 past the batch kernel
+    (4, 4, 4, 1024, 1024, True),     # one chunk of either width, filled; groups of 1 and 3
+    (10, 4, 4, 1008, 528, True),     # groups of 1, 4, 4 and 1
+    (6, 4, 4, 1024, 1040, True),     # a second chunk of the inter width alone
     (64, 4, 4, 4096, 144, True),     # the widest rows, every token on every expert, a down item a resident wave
     (20, 96, 8, 3072, 2048, False),  # bf16, four chunks, the widest inter
     (40, 32, 12, 512, 1024, True),   # A = 480; combine past eight slots
