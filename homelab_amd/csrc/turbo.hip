@@ -203,16 +203,16 @@ __global__ void __launch_bounds__(64 * TR_WAVES) kv_append_kernel(const float* _
 #pragma unroll
     for (int i = 0; i < 4; i++) idx[i] = fabsf(u[i] - lv[idx[i]]) <= fabsf(u[i] - lv[idx[i] + 1]) ? idx[i] : idx[i] + 1;
     // word j of the block: bit t = 4 (l % 8) + i is bit j of coordinate t's code; the 8
-    // lanes OR their nibbles together and lane l % 8 == j keeps word j (in pairs, so that the
-    // words' exchanges overlap; all eight whatever `bits` took 28.5 us for 40000 rows of 256 at 2
-    // bits, one at a time 25.1, pairs 22.3; at 8 bits 36.9, 41.1 and 35.8)
+    // lanes OR their nibbles together and lane l % 8 == j keeps word j (in fours, so that the
+    // words' exchanges overlap; 40000 rows of 256 at 2, 4 and 8 bits: one word at a time 24.6,
+    // 29.5 and 40.6 us, all eight whatever `bits` 28.3, 30.5 and 36.6, fours 23.7, 26.0 and 35.6)
     const int lb = l & 7, b = l >> 3;
     uint32_t mine = 0;
 #pragma unroll
-    for (int j0 = 0; j0 < 8; j0 += 2) {
+    for (int j0 = 0; j0 < 8; j0 += 4) {
         if (j0 >= bits) break;
 #pragma unroll
-        for (int j = j0; j < j0 + 2; j++) {
+        for (int j = j0; j < j0 + 4; j++) {
             uint32_t nib = 0;
 #pragma unroll
             for (int i = 0; i < 4; i++) nib |= (uint32_t)((idx[i] >> j) & 1) << i;
